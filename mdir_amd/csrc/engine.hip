@@ -78,19 +78,6 @@ static T *dupload(const std::vector<T> &v) {
   return p;
 }
 
-static std::vector<int> radices(int K) {
-  std::vector<int> r;
-  int rest = K;
-  for (int f : {8, 4, 2, 3, 5, 7})
-    while (rest % f == 0) {
-      r.push_back(f);
-      rest /= f;
-    }
-  if (rest != 1 || (int)r.size() > kMaxRadices)
-    throw HipError("FFT length " + std::to_string(K) + " has a factor other than 2, 3, 5, 7");
-  return r;
-}
-
 // Twiddles exp(-2 pi i m / K), m < K, rounded once from f64.
 template <typename T>
 struct FftTables {
@@ -105,10 +92,8 @@ struct FftTables {
       h[m] = {(T)cos(a), (T)sin(a)};
     }
     tw = dupload(h);
-    std::vector<int> r = radices(K);
-    axis.K = K;
-    axis.nrad = (int)r.size();
-    for (int i = 0; i < axis.nrad; ++i) axis.rad[i] = r[i];
+    if (!factor_axis(K, axis))
+      throw HipError("FFT length " + std::to_string(K) + " has a factor other than 2, 3, 5, 7");
     axis.tw = tw;
   }
   void release() { dfree(tw); }
@@ -129,7 +114,7 @@ struct Fft3D {
     for (auto &a : ax) a.release();
   }
   static constexpr int TL = tile_lines<T>();
-  size_t lds(int k) const { return (size_t)2 * TL * k * sizeof(cpx<T>); }
+  size_t lds(int k) const { return tile_lds<T>(k); }
   int H() const { return K[2] / 2 + 1; }
   // real (or 64-bit words) -> half spectrum
   void forward(const void *src, bool fixed, cpx<T> *cplx, hipStream_t s) {

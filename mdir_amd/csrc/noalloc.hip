@@ -51,23 +51,6 @@ void *scratch_address() {
   }
   return g_scratch_at[dev];
 }
-
-// Radices of K (8, 4, 2, then 3, 5, 7, the order of the plans' own
-// factorisation, which the kernels' passes follow) into an FftAxis; false
-// when K has another prime factor or too many radices.
-bool factor_axis(int K, FftAxis &ax) {
-  ax.K = K;
-  ax.nrad = 0;
-  int rest = K;
-  const int order[6] = {8, 4, 2, 3, 5, 7};
-  for (int r : order)
-    while (rest % r == 0) {
-      if (ax.nrad == kMaxRadices) return false;
-      ax.rad[ax.nrad++] = r;
-      rest /= r;
-    }
-  return rest == 1;
-}
 }  // namespace
 
 }  // namespace mdhip
@@ -96,7 +79,7 @@ extern "C" int mdrtHipFFTForward3DF32NoAlloc(const float *real, void *complex, i
       at += (size_t)K[a];
     }
     constexpr int TL = Fft3D<float>::TL;
-    auto lds = [](int64_t k) { return (size_t)2 * TL * (size_t)k * sizeof(cpx<float>); };
+    auto lds = [](int64_t k) { return tile_lds<float>((int)k); };
     const int H = (int)(k3 / 2 + 1);
     const int nrows = (int)(k1 * k2);
     cpx<float> *out = static_cast<cpx<float> *>(complex);

@@ -243,7 +243,7 @@ __device__ __forceinline__ void brick_forward_z(const unsigned long long *acc,
   constexpr int R = BrickShape<TL>::R, BY = BrickShape<TL>::BY;
   const int K0 = pp.K[0], K1 = pp.K[1], K2 = pp.K[2], H = K2 / 2 + 1;
   for (int w = threadIdx.x; w < R * K2; w += blockDim.x) {
-    const int rr = w / K2, z = w % K2;
+    const int rr = div_by(w, az.mk), z = w - rr * K2;
     const float v = (float)((double)(long long)acc[w] * kGridUnscale);
     if (rr & 1)
       a[z * TL + (rr >> 1)].y = v;
@@ -251,11 +251,12 @@ __device__ __forceinline__ void brick_forward_z(const unsigned long long *acc,
       a[z * TL + (rr >> 1)].x = v;
   }
   __syncthreads();
-  cpx<float> *res = lds_fft<float, TL>(a, b, az, -1, tw);
+  cpx<float> *res = lds_fft<float, TL, -1>(a, b, az, tw);
+  const uint32_t mh = div_magic((uint32_t)H);
   for (int w = threadIdx.x; w < TL * H; w += blockDim.x) {
-    const int k = w % H, t = w / H;
+    const int t = div_by(w, mh), k = w - t * H;
     const cpx<float> zk = res[k * TL + t];
-    const cpx<float> zm = res[((K2 - k) % K2) * TL + t];
+    const cpx<float> zm = res[(k ? K2 - k : 0) * TL + t];
     const int r1 = 2 * t, r2 = r1 + 1;
     const int ix1 = bx0 + r1 / BY, iy1 = by0 + r1 % BY;
     const int ix2 = bx0 + r2 / BY, iy2 = by0 + r2 % BY;
@@ -396,7 +397,7 @@ __device__ __forceinline__ const cpx<float> *brick_backward_z(
   const int K0 = pp.K[0], K1 = pp.K[1], K2 = pp.K[2], H = K2 / 2 + 1;
   const size_t rows = (size_t)K0 * K1;
   for (int w = threadIdx.x; w < TL * K2; w += blockDim.x) {
-    const int k = w % K2, t = w / K2;
+    const int t = div_by(w, az.mk), k = w - t * K2;
     const int r1 = 2 * t, r2 = r1 + 1;
     const int ix1 = bx0 + r1 / BY, iy1 = by0 + r1 % BY;
     const int ix2 = bx0 + r2 / BY, iy2 = by0 + r2 % BY;
@@ -418,7 +419,7 @@ __device__ __forceinline__ const cpx<float> *brick_backward_z(
                           : cpx<float>{x1.x + x2.y, -x1.y + x2.x};
   }
   __syncthreads();
-  return lds_fft<float, TL>(a, b, az, +1, tw);
+  return lds_fft<float, TL, 1>(a, b, az, tw);
 }
 
 template <int N, int TL>
@@ -462,6 +463,27 @@ __global__ void __launch_bounds__(256) pme_gather_rows(
 template <typename T>
 constexpr int tile_lines() { return sizeof(T) == 4 ? 16 : 8; }
 
+// LDS of a tile of lines of length k: two buffers, and the axis' twiddles
+// where they fit in the 64 KB a launch takes without asking for more (every
+// pass reads them: edges up to 248 in f32).
+template <typename T>
+__host__ __device__ __forceinline__ bool tile_twiddles_fit(int k) {
+  return (size_t)(2 * tile_lines<T>() + 1) * k * sizeof(cpx<T>) <= 65536 - 2048;
+}
+template <typename T>
+inline size_t tile_lds(int k) {
+  return (size_t)(2 * tile_lines<T>() + (tile_twiddles_fit<T>(k) ? 1 : 0)) * k * sizeof(cpx<T>);
+}
+// The twiddles copied to `at`, or the axis' own table; the caller's next
+// barrier orders the copy.
+template <typename T>
+__device__ __forceinline__ const cpx<T> *tile_twiddles(cpx<T> *at, const FftAxis &ax) {
+  const cpx<T> *own = static_cast<const cpx<T> *>(ax.tw);
+  if (!tile_twiddles_fit<T>(ax.K)) return own;
+  for (int w = threadIdx.x; w < ax.K; w += blockDim.x) at[w] = own[w];
+  return at;
+}
+
 // Forward along z of pairs of real rows packed as one complex line, split
 // into the two half spectra.  SRC_FIXED reads (and clears) 64-bit charge
 // words; otherwise a real T grid.
@@ -496,7 +518,7 @@ __global__ void __launch_bounds__(256) fft_rows_r2c(
       a[z * TL + t].x = v;
   }
   __syncthreads();
-  cpx<T> *res = lds_fft<T, TL>(a, b, az, -1);
+  cpx<T> *res = lds_fft<T, TL, -1>(a, b, az);
   for (int w = threadIdx.x; w < TL * H; w += blockDim.x) {
     const int k = w % H, t = w / H;
     const cpx<T> zk = res[k * TL + t];
@@ -542,7 +564,7 @@ __global__ void __launch_bounds__(256) fft_rows_c2r(const cpx<T> *__restrict__ i
     a[k * TL + t] = zv;
   }
   __syncthreads();
-  cpx<T> *res = lds_fft<T, TL>(a, b, az, +1);
+  cpx<T> *res = lds_fft<T, TL, 1>(a, b, az);
   for (int w = threadIdx.x; w < 2 * TL * K; w += blockDim.x) {
     const int z = w % K, rr = w / K;
     const int row = row0 + rr;
@@ -560,6 +582,7 @@ __global__ void __launch_bounds__(256) fft_cols_y(cpx<T> *__restrict__ data, int
   extern __shared__ unsigned char smem[];
   cpx<T> *a = reinterpret_cast<cpx<T> *>(smem);
   cpx<T> *b = a + TL * K2;
+  const cpx<T> *tw = tile_twiddles<T>(b + TL * K2, ay);
   const int tiles = (H + TL - 1) / TL;
   const int i0 = blockIdx.x / tiles, z0 = (blockIdx.x % tiles) * TL;
   cpx<T> *base = data + (size_t)i0 * K2 * H + z0;
@@ -568,7 +591,7 @@ __global__ void __launch_bounds__(256) fft_cols_y(cpx<T> *__restrict__ data, int
     a[y * TL + t] = (z0 + t < H) ? base[(size_t)y * H + t] : cpx<T>{(T)0, (T)0};
   }
   __syncthreads();
-  cpx<T> *res = lds_fft<T, TL>(a, b, ay, sign);
+  cpx<T> *res = sign < 0 ? lds_fft<T, TL, -1>(a, b, ay, tw) : lds_fft<T, TL, 1>(a, b, ay, tw);
   for (int w = threadIdx.x; w < TL * K2; w += blockDim.x) {
     const int t = w % TL, y = w / TL;
     if (z0 + t < H) base[(size_t)y * H + t] = res[y * TL + t];
@@ -595,6 +618,7 @@ __global__ void __launch_bounds__(256) fft_x_conv(cpx<T> *__restrict__ data, int
   extern __shared__ unsigned char smem[];
   cpx<T> *a = reinterpret_cast<cpx<T> *>(smem);
   cpx<T> *b = a + TL * K1;
+  const cpx<T> *tw = tile_twiddles<T>(b + TL * K1, ax);
   __shared__ double s_e[256];
   const int tiles = (H + TL - 1) / TL;
   const int i1 = blockIdx.x / tiles, z0 = (blockIdx.x % tiles) * TL;
@@ -606,7 +630,7 @@ __global__ void __launch_bounds__(256) fft_x_conv(cpx<T> *__restrict__ data, int
   }
   __syncthreads();
   if (mode == -1 || mode == 1) {  // single direction: -1 forward, +1 backward
-    cpx<T> *res = lds_fft<T, TL>(a, b, ax, mode);
+    cpx<T> *res = mode < 0 ? lds_fft<T, TL, -1>(a, b, ax, tw) : lds_fft<T, TL, 1>(a, b, ax, tw);
     for (int w = threadIdx.x; w < TL * K1; w += blockDim.x) {
       const int t = w % TL, xx = w / TL;
       if (z0 + t < H) base[xx * stride + t] = res[xx * TL + t];
@@ -615,7 +639,7 @@ __global__ void __launch_bounds__(256) fft_x_conv(cpx<T> *__restrict__ data, int
   }
   // mode 0: forward, product, backward; mode 2: product, backward (the
   // spectrum is already transformed along x)
-  cpx<T> *res = mode == 0 ? lds_fft<T, TL>(a, b, ax, -1) : a;
+  cpx<T> *res = mode == 0 ? lds_fft<T, TL, -1>(a, b, ax, tw) : a;
   const T *t0 = (const T *)ct.t[0], *t1 = (const T *)ct.t[1], *t2 = (const T *)ct.t[2];
   const T *m0 = (const T *)ct.m[0], *m1 = (const T *)ct.m[1], *m2 = (const T *)ct.m[2];
   double e = 0.0;
@@ -636,7 +660,7 @@ __global__ void __launch_bounds__(256) fft_x_conv(cpx<T> *__restrict__ data, int
   }
   __syncthreads();
   cpx<T> *other = (res == a) ? b : a;
-  cpx<T> *res2 = lds_fft<T, TL>(res, other, ax, +1);
+  cpx<T> *res2 = lds_fft<T, TL, 1>(res, other, ax, tw);
   for (int w = threadIdx.x; w < TL * K1; w += blockDim.x) {
     const int t = w % TL, xx = w / TL;
     if (z0 + t < H) base[xx * stride + t] = res2[xx * TL + t];
@@ -686,10 +710,16 @@ __global__ void __launch_bounds__(512) fft_plane_conv(cpx<float> *__restrict__ d
   const int kz = blockIdx.x;
   cpx<float> *plane = data + (size_t)kz * np;
   const int swz = K2 % 16 == 0 ? 15 : 0;
+  // element w of the plane: its x, y and place in LDS
+  auto at = [&](int w, int &x, int &y) {
+    x = CK2 > 0 ? w / CK2 : div_by(w, ay.mk);
+    y = w - x * K2;
+    return plane_index(x, y, K2, swz);
+  };
+  int kx, ky;
   // the plane (unrolled, so that the loads are issued together)
 #pragma unroll 8
-  for (int w = threadIdx.x; w < np; w += blockDim.x)
-    a[plane_index(w / K2, w % K2, K2, swz)] = plane[w];
+  for (int w = threadIdx.x; w < np; w += blockDim.x) a[at(w, kx, ky)] = plane[w];
   // twiddles and influence tables in LDS: every pass reads them
   for (int w = threadIdx.x; w < K1; w += blockDim.x) {
     s_twx[w] = static_cast<const cpx<float> *>(ax.tw)[w];
@@ -704,11 +734,11 @@ __global__ void __launch_bounds__(512) fft_plane_conv(cpx<float> *__restrict__ d
   __syncthreads();
   cpx<float> *r;
   if constexpr (CK1 > 0) {
-    r = lds_fft_plane_k<float, 1, CK1, CK2>(a, b, -1, swz, s_twy);
-    r = lds_fft_plane_k<float, 0, CK1, CK2>(r, r == a ? b : a, -1, swz, s_twx);
+    r = lds_fft_plane_k<float, 1, -1, CK1, CK2>(a, b, swz, s_twy);
+    r = lds_fft_plane_k<float, 0, -1, CK1, CK2>(r, r == a ? b : a, swz, s_twx);
   } else {
-    r = lds_fft_plane<float, 1>(a, b, ay, -1, K1, K2, swz, s_twy);
-    r = lds_fft_plane<float, 0>(r, r == a ? b : a, ax, -1, K1, K2, swz, s_twx);
+    r = lds_fft_plane<float, 1, -1>(a, b, ay, K1, K2, swz, ay.mk, s_twy);
+    r = lds_fft_plane<float, 0, -1>(r, r == a ? b : a, ax, K1, K2, swz, ay.mk, s_twx);
   }
   const float t2 = static_cast<const float *>(ct.t[2])[kz];
   const float m2 = static_cast<const float *>(ct.m[2])[kz];
@@ -718,8 +748,7 @@ __global__ void __launch_bounds__(512) fft_plane_conv(cpx<float> *__restrict__ d
   // (05-electrostatics.md:262-279): xx yy zz xy xz yz
   double vir[6] = {0, 0, 0, 0, 0, 0};
   for (int w = threadIdx.x; w < np; w += blockDim.x) {
-    const int kx = w / K2, ky = w % K2;
-    const int i = plane_index(kx, ky, K2, swz);
+    const int i = at(w, kx, ky);
     const cpx<float> v = r[i];
     float bc = 0.0f;
     if ((kx | ky | kz) != 0) {
@@ -744,14 +773,14 @@ __global__ void __launch_bounds__(512) fft_plane_conv(cpx<float> *__restrict__ d
   }
   __syncthreads();
   if constexpr (CK1 > 0) {
-    r = lds_fft_plane_k<float, 0, CK1, CK2>(r, r == a ? b : a, +1, swz, s_twx);
-    r = lds_fft_plane_k<float, 1, CK1, CK2>(r, r == a ? b : a, +1, swz, s_twy);
+    r = lds_fft_plane_k<float, 0, 1, CK1, CK2>(r, r == a ? b : a, swz, s_twx);
+    r = lds_fft_plane_k<float, 1, 1, CK1, CK2>(r, r == a ? b : a, swz, s_twy);
   } else {
-    r = lds_fft_plane<float, 0>(r, r == a ? b : a, ax, +1, K1, K2, swz, s_twx);
-    r = lds_fft_plane<float, 1>(r, r == a ? b : a, ay, +1, K1, K2, swz, s_twy);
+    r = lds_fft_plane<float, 0, 1>(r, r == a ? b : a, ax, K1, K2, swz, ay.mk, s_twx);
+    r = lds_fft_plane<float, 1, 1>(r, r == a ? b : a, ay, K1, K2, swz, ay.mk, s_twy);
   }
   for (int w = threadIdx.x; w < np; w += blockDim.x)
-    plane[w] = r[plane_index(w / K2, w % K2, K2, swz)];
+    plane[w] = r[at(w, kx, ky)];
   if (energy_partial) {
     s_e[threadIdx.x] = e;
     __syncthreads();
