@@ -277,6 +277,7 @@ struct Engine {
 
   // ---- integration ----
   int *d_unit_first = nullptr, *d_unit_size = nullptr;
+  int unit_width = 3;  // atoms a unit of d_unit_first may hold
   IntParams ip{};
 
   // ---- Langevin thermostat ----
@@ -284,14 +285,14 @@ struct Engine {
   // (K) with the noise of (seed, step number, atom); 0: velocity Verlet.
   double lv_friction = 0.0, lv_temperature = 0.0;
   unsigned long long lv_seed = 0;
-  long long *d_lstep = nullptr;   // [0] step number of the next step, [1] blocks done
+  long long *d_lstep = nullptr;   // the step number of the next step
   int64_t step_count = 0;         // steps taken: the step number of the next step
   void set_langevin(double temperature, double friction, unsigned long long seed) {
     if (friction < 0.0 || !(temperature >= 0.0)) throw HipError("Langevin: friction and temperature must not be negative");
     lv_friction = friction;
     lv_temperature = temperature;
     lv_seed = seed;
-    if (friction > 0.0 && !d_lstep) d_lstep = dalloc<long long>(2);
+    if (friction > 0.0 && !d_lstep) d_lstep = dalloc<long long>(1);
     invalidate_graph();  // captured graphs hold the integration parameters
   }
   // ---- Monte Carlo barostat ----
@@ -419,8 +420,8 @@ struct Engine {
   // set to the host's count before a chunk of steps.
   void put_step_count() {
     if (!(lv_friction > 0.0)) return;
-    const long long h[2] = {(long long)step_count, 0};
-    to_device(d_lstep, h, sizeof(h));
+    const long long h = (long long)step_count;
+    to_device(d_lstep, &h, sizeof(h));
   }
 
   // ---- checkpoints ----
@@ -1050,6 +1051,7 @@ struct Engine {
           us.push_back(1);
         }
       nunits = (int)uf.size();
+      unit_width = d->nwaters > 0 ? 3 : 1;
       d_unit_first = dupload(uf);
       d_unit_size = dupload(us);
       for (int k = 0; k < 3; ++k) ip.half_box[k] = 0.5 * box[k];
@@ -1631,20 +1633,41 @@ struct Engine {
     } else {
       ip.step = nullptr;
     }
-    if (nclusters)
-      integrate_clusters<PART><<<blocks_for(nclusters, 64), 64, 0, stream>>>(
-          nclusters, d_cl_first, d_cl_code, d_x, d_v, d_inv_mass, d_F, d_Fr, d_place_of,
-          d_shift, d_xref, d_q, d_xq, use_origins() ? d_gorig : nullptr,
-          d_xpa ? nullptr : d_xpq, d_xpa, ip, d_flags);
-    // at least one block: its last block advances the Langevin step number
-    integrate_part<PART><<<std::max(blocks_for(nunits, 64), 1), 64, 0, stream>>>(
-        nunits, d_unit_first, d_unit_size, d_x, d_v, d_inv_mass, d_F, d_Fr, d_place_of,
-        d_shift, d_xref, d_q, d_xq, use_origins() ? d_gorig : nullptr,
-        d_xpa ? nullptr : d_xpq, d_xpa, ip, d_flags);
+    IntUnits un{};
+    un.clusters = nclusters;
+    un.cluster_blocks = (nclusters + kClusterUnits - 1) / kClusterUnits;
+    un.cluster_first = d_cl_first;
+    un.cluster_code = d_cl_code;
+    un.units = nunits;
+    un.width = unit_width;
+    un.first = d_unit_first;
+    un.code = d_unit_size;
+    // constraint clusters are laid out for kIntThreads
+    const int threads = un.width == 1 && !nclusters ? 64 : kIntThreads;
+    un.per_block = threads / un.width;
+    // at least one block: the closing launch advances the step number
+    const int blocks =
+        std::max(un.cluster_blocks + (nunits + un.per_block - 1) / un.per_block, 1);
+    const auto kernel = nclusters ? integrate_units<PART, true> : integrate_units<PART, false>;
+    kernel<<<blocks, threads, 0, stream>>>(un, d_x, d_v, d_inv_mass, d_F, d_Fr, d_place_of,
+                                               d_shift, d_xref, d_q, d_xq,
+                                               use_origins() ? d_gorig : nullptr,
+                                               d_xpa ? nullptr : d_xpq, d_xpa, ip, d_flags);
   }
-  void step_first(double dt) { integrate<kFirstHalf>(dt); }
-  void step_second(double dt) { integrate<kSecondHalf>(dt); }
-  void step_between(double dt) { integrate<kBetween>(dt); }
+  void step_first(double dt) {
+    ip.offset = 0;
+    integrate<kFirstHalf>(dt);
+  }
+  // closes a sequence of `steps` steps
+  void step_second(double dt, int steps) {
+    ip.advance = steps;
+    integrate<kSecondHalf>(dt);
+  }
+  // before step `index` (from 0) of a sequence
+  void step_between(double dt, int index) {
+    ip.offset = index;
+    integrate<kBetween>(dt);
+  }
 
   // `count` whole steps; between two steps the second half of one and the
   // first half of the next run as one kernel.
@@ -1653,8 +1676,8 @@ struct Engine {
     step_first(dt);
     for (int64_t s = 0; s < count; ++s) {
       forces(false, measure ? (int)s : -1, true);
-      if (s + 1 < count) step_between(dt);
-      else step_second(dt);
+      if (s + 1 < count) step_between(dt, (int)(s + 1));
+      else step_second(dt, (int)count);
     }
   }
 
@@ -2262,7 +2285,7 @@ struct Engine {
       HIPCHK(hipEventRecord(ev[k++], stream));
       if (use_pme) pme_gather_rows_launch();
       HIPCHK(hipEventRecord(ev[k++], stream));
-      step_second(0.002);
+      step_second(0.002, 1);
       HIPCHK(hipEventRecord(ev[k++], stream));
       HIPCHK(hipEventSynchronize(ev[kProfileSlots]));
       for (int j = 0; j < kProfileSlots; ++j) {

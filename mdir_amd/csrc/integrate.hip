@@ -9,9 +9,10 @@
 //   (ConstraintIR.cpp:392-471).
 // A unit is a SETTLE water (3 consecutive atoms), a constraint cluster (an
 // atom and up to four atoms bonded to it at fixed lengths, consecutive,
-// M-SHAKE as ConstraintIR.cpp:595-747 takes it) or a free atom; one thread
-// owns a unit, reads its force words and clears them for the next step.
-// Blocks of 64 threads: a few thousand units still spread over every CU.
+// M-SHAKE as ConstraintIR.cpp:595-747 takes it) or a free atom.  A block
+// takes the atoms of its units a thread per atom (loads, half kick, noise,
+// stores; the whole step of a free atom) and their constraints a thread per
+// unit, through LDS (integrate_units).
 #include "md_common.h"
 
 namespace mdhip {
@@ -34,12 +35,14 @@ struct IntParams {
   // Langevin dynamics (langevin != 0): the g-BAOAB step with the O step
   // v <- decay v + spread / sqrt(m) R, decay = exp(-gamma dt) and
   // spread = sqrt((1 - decay^2) kB T); R from langevin_normals(seed, step,
-  // atom).  step[0] is the step number the next first half takes (the
-  // launch's last block advances it), step[1] counts finished blocks.
+  // atom).  A first half takes step number *step + offset; the launch that
+  // closes a sequence of steps adds `advance`, their count, to *step (no
+  // launch that reads the number runs beside it).
   int langevin;
   double decay, spread;
   unsigned long long seed;
   long long *step;
+  int offset, advance;
   // constraint clusters: each member's bond length to its centre, by atom,
   // and the inverse masses (the descent step of a minimisation)
   const double *clen;
@@ -167,36 +170,37 @@ __device__ void settle_velocities(const double *xa, const double *xb, const doub
 }
 
 // The state of one unit of S atoms (a SETTLE water, S = 3, a constraint
-// cluster, S = 2..5, with its centre at index 0, or a free atom, S = 1) in
-// registers: S is a compile-time constant so that the arrays stay in
-// registers.  at[m] is the atom of index m.
+// cluster, S = 2..5, with its centre at index 0) in registers: S is a compile-time constant so that the arrays stay in
+// registers.
 template <int S>
 struct UnitState {
-  int at[S];
-  int pl[S];
-  double im[S], x[S][3], v[S][3], f[S][3];
+  double im[S], x[S][3], v[S][3];
   double len[S];  // clusters: index m's bond length to the centre
 };
 
 // Linear equations A y = b of at most 4 unknowns by elimination (the
-// cluster equations are diagonally dominant: no pivoting).
+// cluster equations are diagonally dominant: no pivoting).  One reciprocal
+// per pivot: a chain of f64 divisions is what a sweep waits for.
 template <int M>
 __device__ __forceinline__ void solve_small(double (&A)[M][M], double (&b)[M]) {
+  double inv[M];
 #pragma unroll
-  for (int i = 0; i < M; ++i)
+  for (int i = 0; i < M; ++i) {
+    inv[i] = 1.0 / A[i][i];
 #pragma unroll
     for (int r = i + 1; r < M; ++r) {
-      const double f = A[r][i] / A[i][i];
+      const double f = A[r][i] * inv[i];
 #pragma unroll
       for (int c = i; c < M; ++c) A[r][c] -= f * A[i][c];
       b[r] -= f * b[i];
     }
+  }
 #pragma unroll
   for (int i = M - 1; i >= 0; --i) {
     double sum = b[i];
 #pragma unroll
     for (int c = i + 1; c < M; ++c) sum -= A[i][c] * b[c];
-    b[i] = sum / A[i][i];
+    b[i] = sum * inv[i];
   }
 }
 
@@ -271,49 +275,15 @@ __device__ __forceinline__ void rattle_velocities(const double (&x)[S][3], doubl
     }
 }
 
-// Loads the unit at `first`; with clear, the force words are zeroed for the
-// next evaluation once read.  Fr (or null): reciprocal force words by atom,
-// added to the place-ordered words as integers before the conversion, so
-// the force is the one a single word would hold.
-template <int S, bool CL>
-__device__ __forceinline__ void load_unit(int first, int code, const double *__restrict__ x,
-                                          const double *__restrict__ v,
-                                          const double *__restrict__ inv_mass,
-                                          long long *__restrict__ F,
-                                          long long *__restrict__ Fr,
-                                          const int *__restrict__ place_of, bool clear,
-                                          const IntParams &p, UnitState<S> &s) {
-  const int centre = CL ? (code >> kUnitCentreShift) & 15 : 0;
-#pragma unroll
-  for (int m = 0; m < S; ++m) {
-    // clusters: the centre first, then the others in their order
-    const int at = CL ? first + (m == 0 ? centre : (m - 1 < centre ? m - 1 : m)) : first + m;
-    s.at[m] = at;
-    s.len[m] = CL && m > 0 ? p.clen[at] : 0.0;
-    s.pl[m] = place_of[at];
-    s.im[m] = inv_mass[at];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      long long w = F[3 * s.pl[m] + k];
-      if (Fr) {
-        w += Fr[3 * at + k];
-        if (clear) Fr[3 * at + k] = 0;
-      }
-      s.f[m][k] = (double)w * kForceUnscale;
-      if (clear) F[3 * s.pl[m] + k] = 0;
-      s.v[m][k] = v[3 * at + k];
-      s.x[m][k] = x[3 * at + k];
-    }
-  }
-}
-
-template <int S>
-__device__ __forceinline__ void half_kick(UnitState<S> &s, double dt) {
-#pragma unroll
-  for (int m = 0; m < S; ++m)
-#pragma unroll
-    for (int k = 0; k < 3; ++k) s.v[m][k] = s.v[m][k] + 0.5 * dt * s.f[m][k] * s.im[m];
-}
+// The atoms of a block's units in LDS, slot t of every array belonging to
+// thread t (a unit's members are consecutive slots): positions, velocities,
+// the half kick dt/2 f/m, the noise spread/sqrt(m) R of a Langevin step, the
+// inverse masses and the bond lengths.
+constexpr int kIntThreads = 192;
+struct UnitLds {
+  double x[3][kIntThreads], v[3][kIntThreads], kick[3][kIntThreads], noise[3][kIntThreads];
+  double im[kIntThreads], len[kIntThreads];
+};
 
 template <int S, bool CL>
 __device__ __forceinline__ void constrain_velocities(UnitState<S> &s, const double (&x)[S][3],
@@ -348,118 +318,90 @@ __device__ __forceinline__ void drift_settle(const UnitState<S> &s, const double
   }
 }
 
-// The rest of a g-BAOAB step after its first half kick (B): the geodesic
-// integrator of Leimkuhler and Matthews (Proc. R. Soc. A 472, 20160138,
-// 2016), as the reference's Langevin step with constraints takes it
-// (lib/Driver/DynamicsIR.cpp, the geodesic branch): project v onto the
-// constraints; A: half drift, SETTLE, v += dx_c / (dt/2); O: v <- decay v +
-// spread / sqrt(m) R, projected again at the new positions; A: half drift
-// from there, SETTLE, v += dx_c / (dt/2).  The closing B (kick and
-// projection) is the second half of the step, as in velocity Verlet.
-template <int S, bool CL>
-__device__ __forceinline__ void baoab_rest(UnitState<S> &s, double (&xn)[S][3], long long step,
-                                           const IntParams &p) {
-  const double h = 0.5 * p.dt;
-  constrain_velocities<S, CL>(s, s.x, p);
-  double xh[S][3];
-  drift_settle<S, CL>(s, s.x, s.v, xh, h, p);
-#pragma unroll
-  for (int m = 0; m < S; ++m) {
-    if (!(s.im[m] > 0.0)) continue;  // a particle without mass keeps its velocity
-    double r[3];
-    langevin_normals(p.seed, step, (uint32_t)s.at[m], r);
-    const double width = p.spread * sqrt(s.im[m]);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) s.v[m][k] = p.decay * s.v[m][k] + width * r[k];
-  }
-  constrain_velocities<S, CL>(s, xh, p);
-  drift_settle<S, CL>(s, xh, s.v, xn, h, p);
-}
-
-// Stores x, v and the f32 positions of the pair loop after a drift to xn;
-// returns bit 0 when an atom moved beyond half the list buffer since the
-// build, bit 1 beyond half the pruned list's buffer since the last prune.
-template <int S>
-__device__ __forceinline__ int store_drifted(UnitState<S> &s, const double (&xn)[S][3],
-                                             double *__restrict__ x, double *__restrict__ v,
-                                             const double *__restrict__ shift,
-                                             const double *__restrict__ xref,
-                                             const double *__restrict__ q,
-                                             float4 *__restrict__ xq,
-                                             const float4 *__restrict__ gorig,
-                                             double4 *__restrict__ xpq,
-                                             double4 *__restrict__ xpa, const IntParams &p) {
-  int moved = 0;  // bit 0: beyond the list buffer, bit 1: beyond the pruned one
-#pragma unroll
-  for (int m = 0; m < S; ++m) {
-    const int at = s.at[m];
-    double d2 = 0.0, d2p = 0.0;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      x[3 * at + k] = xn[m][k];
-      v[3 * at + k] = s.v[m][k];
-      const double d = xn[m][k] - xref[3 * at + k];
-      d2 += d * d;
-      if (p.x_prune) {
-        const double dp = xn[m][k] - p.x_prune[3 * at + k];
-        d2p += dp * dp;
-      }
-    }
-    if (d2 > p.skin_half2) moved |= 1;
-    if (d2p > p.prune_half2) moved |= 2;
-    const float4 o = gorig ? gorig[s.pl[m] / (kCluster * kGroup)]
-                           : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    xq[s.pl[m]] = make_float4(
-        (float)(xn[m][0] - shift[3 * at + 0] - p.half_box[0] - (double)o.x),
-        (float)(xn[m][1] - shift[3 * at + 1] - p.half_box[1] - (double)o.y),
-        (float)(xn[m][2] - shift[3 * at + 2] - p.half_box[2] - (double)o.z), (float)q[at]);
-    if (xpq) xpq[s.pl[m]] = make_double4(xn[m][0], xn[m][1], xn[m][2], q[at]);
-    if (xpa) xpa[at] = make_double4(xn[m][0], xn[m][1], xn[m][2], q[at]);
-  }
-  return moved;
-}
-
 // Which halves of velocity Verlet a launch runs on each unit.
 enum StepPart { kFirstHalf = 1, kSecondHalf = 2, kBetween = 3 };
 
+// The unit whose members are slots t .. t + S - 1: kicks, constraints and
+// drifts, LDS to LDS.  A step is a sequence of stages, each the velocity
+// constraint at x and then a drift from x:
+//   end of a step (kSecondHalf)   constraint; the kick that starts the next
+//                                 step (kBetween)
+//   velocity Verlet               drift of dt
+//   Langevin                      constraint, drift of dt/2; O step; both
+//                                 again
+// (the g-BAOAB geodesic integrator of Leimkuhler and Matthews, Proc. R. Soc.
+// A 472, 20160138, 2016, as the reference's Langevin step with constraints
+// takes it, lib/Driver/DynamicsIR.cpp, the geodesic branch: project v onto
+// the constraints; A: half drift, SETTLE, v += dx_c / (dt/2); O: v <- decay
+// v + spread / sqrt(m) R, projected again at the new positions; A: half
+// drift from there.  The closing B, kick and projection, is the second half
+// of the step, as in velocity Verlet.)  One loop over the stages holds the
+// constraint and the drift once: the kernel runs its code once per launch,
+// so what it waits for is its instructions' way to the CU.
 template <int PART, int S, bool CL>
-__device__ __forceinline__ void step_unit(int first, int code, long long step,
-                                          double *__restrict__ x,
-                                          double *__restrict__ v,
-                                          const double *__restrict__ inv_mass,
-                                          long long *__restrict__ F,
-                                          long long *__restrict__ Fr,
-                                          const int *__restrict__ place_of,
-                                          const double *__restrict__ shift,
-                                          const double *__restrict__ xref,
-                                          const double *__restrict__ q,
-                                          float4 *__restrict__ xq,
-                                          const float4 *__restrict__ gorig,
-                                          double4 *__restrict__ xpq,
-                                          double4 *__restrict__ xpa, const IntParams &p,
-                                          int *__restrict__ flags) {
+__device__ __forceinline__ void step_unit(UnitLds &l, int t, const IntParams &p) {
   UnitState<S> s;
-  // the force words are cleared by the launch that reads them last
-  load_unit<S, CL>(first, code, x, v, inv_mass, F, Fr, place_of, PART != kSecondHalf, p, s);
-  if (PART & kSecondHalf) {  // end of a step: half kick, velocity constraint
-    half_kick<S>(s, p.dt);
-    constrain_velocities<S, CL>(s, s.x, p);
+#pragma unroll
+  for (int m = 0; m < S; ++m) {
+    s.im[m] = l.im[t + m];
+    s.len[m] = CL ? l.len[t + m] : 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      s.x[m][k] = l.x[k][t + m];
+      s.v[m][k] = l.v[k][t + m] + l.kick[k][t + m];
+    }
   }
-  if (PART & kFirstHalf) {   // start of a step: half kick, drift, constraints
-    half_kick<S>(s, p.dt);
+  const bool langevin = (PART & kFirstHalf) && p.langevin;
+  const int drifts = PART & kFirstHalf ? (langevin ? 2 : 1) : 0;
+  const double h = langevin ? 0.5 * p.dt : p.dt;
+#pragma unroll 1
+  for (int stage = PART & kSecondHalf ? 0 : 1; stage <= drifts; ++stage) {
+    if (stage == 0 || langevin) constrain_velocities<S, CL>(s, s.x, p);
+    if (stage == 0) {
+      if (PART == kBetween) {
+#pragma unroll
+        for (int m = 0; m < S; ++m)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) s.v[m][k] = s.v[m][k] + l.kick[k][t + m];
+      }
+      continue;
+    }
     double xn[S][3];
-    if (p.langevin) baoab_rest<S, CL>(s, xn, step, p);
-    else drift_settle<S, CL>(s, s.x, s.v, xn, p.dt, p);
-    const int moved = store_drifted<S>(s, xn, x, v, shift, xref, q, xq, gorig, xpq, xpa, p);
-    if (moved & 1) atomicOr(&flags[kFlagRebuild], 1);
-    if (moved & 2) atomicOr(&flags[kFlagPrune], 1);
-  } else {
+    drift_settle<S, CL>(s, s.x, s.v, xn, h, p);
 #pragma unroll
     for (int m = 0; m < S; ++m)
 #pragma unroll
-      for (int k = 0; k < 3; ++k) v[3 * s.at[m] + k] = s.v[m][k];
+      for (int k = 0; k < 3; ++k) s.x[m][k] = xn[m][k];
+    if (stage == 1 && langevin) {
+#pragma unroll
+      for (int m = 0; m < S; ++m) {
+        if (!(s.im[m] > 0.0)) continue;  // a particle without mass keeps its velocity
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s.v[m][k] = p.decay * s.v[m][k] + l.noise[k][t + m];
+      }
+    }
   }
+#pragma unroll
+  for (int m = 0; m < S; ++m)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      if (PART & kFirstHalf) l.x[k][t + m] = s.x[m][k];
+      l.v[k][t + m] = s.v[m][k];
+    }
 }
+
+// The units of a launch: `clusters` constraint clusters, kClusterUnits per
+// block, in the first blocks (their solves take longest), then the waters
+// and free atoms, `threads` / width per block: kIntThreads and width 3 with
+// waters, a wave and width 1 in a system of free atoms.
+struct IntUnits {
+  int clusters, cluster_blocks;
+  const int *cluster_first, *cluster_code;
+  int units, width, per_block;   // units per block: threads / width
+  const int *first, *code;
+};
+constexpr int kClusterSlots = 5;
+constexpr int kClusterUnits = kIntThreads / kClusterSlots;
 
 // PART kFirstHalf: half kick with the force words (cleared), drift, SETTLE,
 // v += dx_c/dt, f32 positions of the pair loop, validity flag.
@@ -467,66 +409,176 @@ __device__ __forceinline__ void step_unit(int first, int code, long long step,
 // first half reads them) and the velocity constraint.  kBetween: both, the
 // second half of one step and the first half of the next, in one pass over
 // the state with the same operations in the same order.
-template <int PART>
-__global__ void __launch_bounds__(64) integrate_part(
-    int nunits, const int *__restrict__ unit_first, const int *__restrict__ unit_size,
-    double *__restrict__ x, double *__restrict__ v, const double *__restrict__ inv_mass,
-    long long *__restrict__ F, long long *__restrict__ Fr, const int *__restrict__ place_of,
+//
+// Thread per atom outside the constraints: consecutive threads load and
+// store consecutive atoms, the three atoms of a water draw their noise side
+// by side and while the loads are in flight, and 64 units make three waves
+// of loads.  A thread per unit for all of it took 72-byte strides through
+// every array and its noise in series.  CL: with constraint clusters (their
+// solves take more registers).
+//
+// A launch is bound by its latencies (load, constraints, store) up to some
+// 100,000 atoms and by memory beyond.  Langevin steps between two steps,
+// a launch alone: 11.9 us at 14,000 atoms (a thread per unit, with a step
+// counter that every block advanced behind a fence: 18.2), 90 us at
+// 999,000 (520; 300 bytes an atom, 3.3 TB/s); 9.5 us without noise at
+// 24,000 (11.8).
+template <int PART, bool CL>
+__global__ void __launch_bounds__(kIntThreads) integrate_units(
+    IntUnits un, double *__restrict__ x, double *__restrict__ v,
+    const double *__restrict__ inv_mass, long long *__restrict__ F,
+    long long *__restrict__ Fr, const int *__restrict__ place_of,
     const double *__restrict__ shift, const double *__restrict__ xref,
     const double *__restrict__ q, float4 *__restrict__ xq, const float4 *__restrict__ gorig,
     double4 *__restrict__ xpq, double4 *__restrict__ xpa, IntParams p,
     int *__restrict__ flags) {
-  const int u = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool noise = (PART & kFirstHalf) && p.langevin;
-  const long long step = noise ? p.step[0] : 0;
-  if (u < nunits) {
-    const int first = unit_first[u], code = unit_size[u];
-    if (code == 3)
-      step_unit<PART, 3, false>(first, code, step, x, v, inv_mass, F, Fr, place_of, shift,
-                                xref, q, xq, gorig, xpq, xpa, p, flags);
-    else
-      step_unit<PART, 1, false>(first, code, step, x, v, inv_mass, F, Fr, place_of, shift,
-                                xref, q, xq, gorig, xpq, xpa, p, flags);
-  }
-  if (noise && threadIdx.x == 0) {
-    // every block has read the step number before it counts itself done
-    // (the fence completes this block's loads); the last one advances it
-    __threadfence();
-    unsigned long long *count = reinterpret_cast<unsigned long long *>(p.step + 1);
-    if (atomicAdd(count, 1ull) + 1ull == (unsigned long long)gridDim.x) {
-      p.step[0] = step + 1;
-      p.step[1] = 0;
+  __shared__ UnitLds l;
+  const int t = threadIdx.x;
+  const bool cluster = CL && (int)blockIdx.x < un.cluster_blocks;
+  const int block = blockIdx.x - (CL && !cluster ? un.cluster_blocks : 0);
+  const int width = cluster ? kClusterSlots : un.width;
+  const int per_block = cluster ? kClusterUnits : un.per_block;
+  const int count = cluster ? un.clusters : un.units;
+  const int *__restrict__ ufirst = cluster ? un.cluster_first : un.first;
+  const int *__restrict__ ucode = cluster ? un.cluster_code : un.code;
+  if (PART == kSecondHalf && p.langevin && blockIdx.x == 0 && t == 0) *p.step += p.advance;
+
+  // this thread's atom
+  const int ul = cluster ? t / kClusterSlots : (width == 3 ? t / 3 : t), m = t - ul * width;
+  const int u = block * per_block + ul;
+  int at = -1;
+  bool free = false;   // a free atom: its thread takes it through the step
+  if (ul < per_block && u < count) {
+    const int first = ufirst[u], code = ucode[u];
+    free = code == 1;
+    if (m < (code & 0xff)) {
+      // clusters: the centre first, then the others in their order
+      const int centre = (code >> kUnitCentreShift) & 15;
+      at = cluster ? first + (m == 0 ? centre : (m - 1 < centre ? m - 1 : m)) : first + m;
     }
   }
-}
-
-// The same parts for the constraint clusters, a launch of their own (their
-// solves would raise the water kernel's registers): launched before
-// integrate_part on the same stream, it reads the step number and leaves
-// its advance to integrate_part.
-template <int PART>
-__global__ void __launch_bounds__(64) integrate_clusters(
-    int nclusters, const int *__restrict__ cluster_first, const int *__restrict__ cluster_code,
-    double *__restrict__ x, double *__restrict__ v, const double *__restrict__ inv_mass,
-    long long *__restrict__ F, long long *__restrict__ Fr, const int *__restrict__ place_of,
-    const double *__restrict__ shift, const double *__restrict__ xref,
-    const double *__restrict__ q, float4 *__restrict__ xq, const float4 *__restrict__ gorig,
-    double4 *__restrict__ xpq, double4 *__restrict__ xpa, IntParams p,
-    int *__restrict__ flags) {
-  const int u = blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= nclusters) return;
-  const long long step = (PART & kFirstHalf) && p.langevin ? p.step[0] : 0;
-  const int first = cluster_first[u], code = cluster_code[u];
-#define STEP_CLUSTER(S)                                                                     \
-  step_unit<PART, S, true>(first, code, step, x, v, inv_mass, F, Fr, place_of, shift, xref, q, \
-                           xq, gorig, xpq, xpa, p, flags)
-  switch (code & 0xff) {
-    case 2: STEP_CLUSTER(2); break;
-    case 3: STEP_CLUSTER(3); break;
-    case 4: STEP_CLUSTER(4); break;
-    default: STEP_CLUSTER(5); break;
+  int pl = 0;
+  double xa[3], va[3], sh[3], xr[3], xp[3], qa = 0.0;
+  float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (at >= 0) {
+    pl = place_of[at];
+    const double im = inv_mass[at];
+    long long w[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      w[k] = Fr ? Fr[3 * at + k] : 0;
+      va[k] = v[3 * at + k];
+      xa[k] = x[3 * at + k];
+      if (PART & kFirstHalf) {
+        sh[k] = shift[3 * at + k];
+        xr[k] = xref[3 * at + k];
+        xp[k] = p.x_prune ? p.x_prune[3 * at + k] : 0.0;
+      }
+    }
+    if (PART & kFirstHalf) {
+      qa = q[at];
+      if (gorig) o = gorig[pl / (kCluster * kGroup)];
+    }
+    // Fr (or null): reciprocal force words by atom, added to the
+    // place-ordered words as integers before the conversion, so the force
+    // is the one a single word would hold.  The words are cleared by the
+    // launch that reads them last.
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      w[k] += F[3 * pl + k];
+      if (PART != kSecondHalf) {
+        F[3 * pl + k] = 0;
+        if (Fr) Fr[3 * at + k] = 0;
+      }
+    }
+    double kick[3], noise[3] = {0.0, 0.0, 0.0};
+    if ((PART & kFirstHalf) && p.langevin && im > 0.0) {
+      langevin_normals(p.seed, *p.step + p.offset, (uint32_t)at, noise);
+      const double spread = p.spread * sqrt(im);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) noise[k] = spread * noise[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) kick[k] = 0.5 * p.dt * ((double)w[k] * kForceUnscale) * im;
+    if (free) {  // step_unit without constraints
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        va[k] = va[k] + kick[k];
+        if (PART == kBetween) va[k] = va[k] + kick[k];
+        if ((PART & kFirstHalf) && p.langevin) {
+          const double h = 0.5 * p.dt;
+          xa[k] = xa[k] + h * va[k];
+          if (im > 0.0) va[k] = p.decay * va[k] + noise[k];
+          xa[k] = xa[k] + h * va[k];
+        } else if (PART & kFirstHalf) {
+          xa[k] = xa[k] + p.dt * va[k];
+        }
+      }
+    } else {
+      l.im[t] = im;
+      if (cluster) l.len[t] = m > 0 ? p.clen[at] : 0.0;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        l.x[k][t] = xa[k];
+        l.v[k][t] = va[k];
+        l.kick[k][t] = kick[k];
+        l.noise[k][t] = noise[k];
+      }
+    }
   }
-#undef STEP_CLUSTER
+  if (width > 1) {
+    __syncthreads();
+    // this thread's unit
+    const int mine = block * per_block + t;
+    if (t < per_block && mine < count) {
+      const int code = ucode[mine], t0 = t * width;
+      if (cluster) {
+        if constexpr (CL) {
+          switch (code & 0xff) {
+            case 2: step_unit<PART, 2, true>(l, t0, p); break;
+            case 3: step_unit<PART, 3, true>(l, t0, p); break;
+            case 4: step_unit<PART, 4, true>(l, t0, p); break;
+            default: step_unit<PART, 5, true>(l, t0, p); break;
+          }
+        }
+      } else if (code == 3) {
+        step_unit<PART, 3, false>(l, t0, p);
+      }
+    }
+    __syncthreads();
+  }
+  if (at < 0) return;
+  if (!free) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      xa[k] = l.x[k][t];
+      va[k] = l.v[k][t];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) v[3 * at + k] = va[k];
+  if (PART & kFirstHalf) {
+    double d2 = 0.0, d2p = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      x[3 * at + k] = xa[k];
+      const double d = xa[k] - xr[k];
+      d2 += d * d;
+      if (p.x_prune) {
+        const double dp = xa[k] - xp[k];
+        d2p += dp * dp;
+      }
+    }
+    // beyond half the list's buffer since the build, beyond half the pruned
+    // list's since the last prune
+    if (d2 > p.skin_half2) atomicOr(&flags[kFlagRebuild], 1);
+    if (d2p > p.prune_half2) atomicOr(&flags[kFlagPrune], 1);
+    xq[pl] = make_float4((float)(xa[0] - sh[0] - p.half_box[0] - (double)o.x),
+                         (float)(xa[1] - sh[1] - p.half_box[1] - (double)o.y),
+                         (float)(xa[2] - sh[2] - p.half_box[2] - (double)o.z), (float)qa);
+    if (xpq) xpq[pl] = make_double4(xa[0], xa[1], xa[2], qa);
+    if (xpa) xpa[at] = make_double4(xa[0], xa[1], xa[2], qa);
+  }
 }
 
 // The isotropic or axis-wise scaling of a Monte Carlo volume move: each
