@@ -222,11 +222,33 @@ struct Engine {
   int *d_row_count_in = nullptr;
   double *d_xprune = nullptr;      // positions at the last prune
   int ex_cap = 0;
-  int max_groups = 0, nseg = 0;    // group rows; pair-loop segments per row
+  int max_groups = 0;              // group rows
   // entries per pair-loop segment (16, 24 or 48): short segments give one
   // system more waves to hide latency with; a batch of frames fills the
   // GPU with long ones (a launch shape, see autotune)
   int seg_len = 16, seg_len_cfg = 0;
+  // Entries one wave of the pair loops takes ("piece"): the segment, halved
+  // (down to kPieceMin) while the launch would hold fewer than kFillPieces
+  // pieces.  A wave walks its entries in series, and a small box has fewer
+  // waves than the GPU has SIMDs: 864 argon atoms took 11.9 us for 16
+  // entries (50 steps 1,060 us), 4 entries take the 50 steps to 810 us.
+  // Pieces are counted by capacity, about three times the entries the rows
+  // hold: the line lies near 1,000 waters, below which PME is shorter than
+  // the pair loop.  A line at 16,384 (4,000 waters) gave nothing more alone
+  // and cost replicas, which share the GPU, 2 to 4 %.  Frame batches keep
+  // whole segments: a frame's forces have the same bits whatever batch it
+  // is in, and the sums over a piece are f32.
+  static constexpr int kPieceMin = 4;
+  static constexpr double kFillPieces = 4096;
+  bool split_segments = true;
+  int piece() const {
+    int len = seg_len;
+    while (split_segments && len / 2 >= kPieceMin &&
+           (double)max_groups * g.row_cap / len < kFillPieces)
+      len /= 2;
+    return len;
+  }
+  int nseg() const { return (g.row_cap + piece() - 1) / piece(); }  // pieces per row
   int *d_excl_start = nullptr, *d_excl_atoms = nullptr;
   int *d_flags = nullptr;
   double list_reach = 0;  // rlist of the current list configuration
@@ -736,7 +758,6 @@ struct Engine {
     list_reach = reach;
     if (same) return;
     max_groups = ngroups_max;
-    nseg = g.row_cap / seg_len;
     seg_len_cfg = seg_len;
     ex_cap = nex;
     release_list();
@@ -765,7 +786,7 @@ struct Engine {
       d_rows_in = dalloc<PairEntry>((size_t)max_groups * g.row_cap);
       d_row_count_in = dalloc<int>(max_groups);
     }
-    d_epair = dalloc<double>(2 * (size_t)max_groups * nseg);
+    d_epair = dalloc<double>(2 * (size_t)max_groups * nseg());
     forces_valid = false;
     invalidate_graph();
   }
@@ -1232,23 +1253,23 @@ struct Engine {
       bonded_tuples<<<tb, 256, 0, lstream>>>(ta, d_x, d_place_of, box[0], box[1], box[2], d_F);
     }
     const dim3 grid(std::max(blocks_for(max_groups, 4), blocks_for(nspecial)),
-                    (terms & 1) ? nseg + 1 : 1, nz);
+                    (terms & 1) ? nseg() + 1 : 1, nz);
     const bool pruned = prune_skin > 0;
     const size_t lds = ntypes * ntypes * sizeof(float2);
     if constexpr (ORG)
       nb_pairs_org<MOD, COUL, ENERGY><<<grid, 256, lds, lstream>>>(
           d_xq, d_gorig, d_type_at, d_real_mask, pruned ? d_rows_in : d_rows,
-          pruned ? d_row_count_in : d_row_count, d_ex, g.row_cap, seg_len, max_groups, d_counts,
+          pruned ? d_row_count_in : d_row_count, d_ex, g.row_cap, piece(), max_groups, d_counts,
           d_lj, nbp, d_F, d_epair, d_flags, sa, fs);
     else if (nz > 1)  // a batch of frames
       nb_pairs_batch<MOD, COUL, ENERGY><<<grid, 256, lds, lstream>>>(
           d_xq, d_gorig, d_type_at, d_real_mask, pruned ? d_rows_in : d_rows,
-          pruned ? d_row_count_in : d_row_count, d_ex, g.row_cap, seg_len, max_groups, d_counts,
+          pruned ? d_row_count_in : d_row_count, d_ex, g.row_cap, piece(), max_groups, d_counts,
           d_lj, nbp, d_F, d_epair, d_flags, sa, fs);
     else
       nb_pairs<MOD, COUL, ENERGY, false><<<grid, 256, lds, lstream>>>(
           d_xq, d_gorig, d_type_at, d_real_mask, pruned ? d_rows_in : d_rows,
-          pruned ? d_row_count_in : d_row_count, d_ex, g.row_cap, seg_len, max_groups, d_counts,
+          pruned ? d_row_count_in : d_row_count, d_ex, g.row_cap, piece(), max_groups, d_counts,
           d_lj, nbp, d_F, d_epair, d_flags, sa, fs);
   }
 
@@ -1803,7 +1824,7 @@ struct Engine {
     if (E_out) {
       for (int k = 0; k < MDRT_NUM_ENERGIES; ++k) E_out[k] = 0.0;
       // one partial per (segment, group) wave, summed in a fixed order
-      std::vector<double> ep(2 * (size_t)max_groups * nseg);
+      std::vector<double> ep(2 * (size_t)max_groups * nseg());
       to_host(ep.data(), d_epair, ep.size() * sizeof(double));
       for (size_t w = 0; (terms & 1) && w < ep.size() / 2; ++w) {
         E_out[MDRT_E_LJ] += ep[2 * w];

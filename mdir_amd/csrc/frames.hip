@@ -70,7 +70,7 @@ struct FrameBatch {
     d_cot = dalloc<float4>(e.max_places);
     d_A = dalloc<long long>(3 * (size_t)e.max_places);
     d_meta = dalloc<double>(4);
-    d_vpart = dalloc<double>((size_t)kPartStride * e.max_groups * e.nseg);
+    d_vpart = dalloc<double>((size_t)kPartStride * e.max_groups * e.nseg());
     d_vspec = dalloc<double>(6 * (size_t)std::max(1, blocks_for(e.nspecial)));
     e.frame_extra = {(void **)&d_fin, (void **)&d_fout, (void **)&d_cot, (void **)&d_A,
                      (void **)&d_meta, (void **)&d_vpart, (void **)&d_vspec};
@@ -92,6 +92,7 @@ struct FrameBatch {
     dd.nwaters = 0;       // no integration
     e.pme_atoms = false;  // the adjoint reads PME inputs in place order
     e.seg_len = 48;       // many frames fill the GPU: long segments
+    e.split_segments = false;
     e.origins_allowed = false;  // the adjoint reads positions about the box centre
     e.create(&dd);
     max_frames = frames;
@@ -296,7 +297,7 @@ struct FrameBatch {
   // Energy terms of every frame (MDRT_NUM_ENERGIES each), partial sums
   // added in a fixed order.
   void frame_energies(int frames, double *out) {
-    const size_t ne = 2 * (size_t)e.max_groups * e.nseg;
+    const size_t ne = 2 * (size_t)e.max_groups * e.nseg();
     std::vector<double> ep((size_t)frames * ne);
     HIPCHK(hipMemcpy2DAsync(ep.data(), ne * sizeof(double), e.d_epair, e.fs, ne * sizeof(double),
                             frames, hipMemcpyDeviceToHost, e.stream));
@@ -343,7 +344,7 @@ struct FrameBatch {
                                 e.stream));
       return v;
     };
-    const size_t np = (size_t)kPartStride * e.max_groups * e.nseg;
+    const size_t np = (size_t)kPartStride * e.max_groups * e.nseg();
     const size_t ns = e.nspecial ? 6 * (size_t)blocks_for(e.nspecial) : 0;
     const size_t nr = e.use_pme ? 6 * (size_t)e.fft.H() : 0;
     const std::vector<double> vp = read(d_vpart, np), vs = read(d_vspec, ns),
@@ -389,14 +390,14 @@ struct FrameBatch {
     sa.rs = e.switch_from;
     for (int k = 0; k < 3; ++k) sa.box[k] = e.box[k];
     sa.lj_modifier = e.lj_modifier;
-    const dim3 grid(std::max(blocks_for(e.max_groups, 4), blocks_for(e.nspecial)), e.nseg + 1,
+    const dim3 grid(std::max(blocks_for(e.max_groups, 4), blocks_for(e.nspecial)), e.nseg() + 1,
                     e.nz);
     const AdjTables tab{d_ljadj, d_ljunit, d_sel};
     const bool parts = KIND == kAdjVirial || KIND == kAdjPairTable;
     const size_t lds = (size_t)e.ntypes * e.ntypes * (sizeof(float4) + sizeof(float2) + sizeof(int));
     nb_adjoint<MOD, COUL, KIND><<<grid, 256, lds, e.stream>>>(
         e.d_xq, e.d_type_at, e.d_real_mask, e.d_rows, e.d_row_count, e.d_ex, e.g.row_cap,
-        e.seg_len, e.max_groups, e.d_counts, tab, ap, d_cot, d_meta, d_A, parts ? d_vpart : nullptr,
+        e.piece(), e.max_groups, e.d_counts, tab, ap, d_cot, d_meta, d_A, parts ? d_vpart : nullptr,
         KIND == kAdjVirial ? d_vspec : nullptr, sa, e.fs);
   }
   template <int KIND>
@@ -597,7 +598,7 @@ struct FrameBatch {
     cot_prepare<<<dim3(1, 1, e.nz), kCotThreads, 0, e.stream>>>(
         0, e.d_counts, e.d_atom_at, e.d_F, d_fin, d_meta, d_cot, e.max_places, e.fs);
     launch_adjoint_k<kAdjPairTable>();
-    const size_t np = (size_t)kPartStride * e.max_groups * e.nseg;
+    const size_t np = (size_t)kPartStride * e.max_groups * e.nseg();
     std::vector<double> vp((size_t)frames * np), meta((size_t)frames * 4);
     HIPCHK(hipMemcpy2DAsync(vp.data(), np * sizeof(double), d_vpart, e.fs, np * sizeof(double),
                             frames, hipMemcpyDeviceToHost, e.stream));
