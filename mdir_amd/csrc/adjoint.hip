@@ -715,9 +715,10 @@ __device__ __forceinline__ void bspline_d2(float w, float *d2) {
 
 // The part of one atom's dipole weights q c . grad W in the brick, added to
 // the brick's accumulators (c in grid units: c_a K_a / L_a).
-template <int N, int BX, int BY>
-__device__ __forceinline__ void spread_dipole_atom(double4 pq, float4 c, const PmeParams &pp,
-                                                   int bx0, int by0, unsigned long long *acc) {
+template <int N, int BX, int BY, int SP>
+__device__ __forceinline__ void spread_dipole_atom(double4 pq, float4 c, int half,
+                                                   const PmeParams &pp, int bx0, int by0,
+                                                   unsigned long long *acc) {
   const int K0 = pp.K[0], K1 = pp.K[1], K2 = pp.K[2];
   int f[3];
   float w[3];
@@ -731,15 +732,24 @@ __device__ __forceinline__ void spread_dipole_atom(double4 pq, float4 c, const P
   const float cx = q * c.x * (float)(K0 * pp.inv_box[0]);
   const float cy = q * c.y * (float)(K1 * pp.inv_box[1]);
   const float cz = q * c.z * (float)(K2 * pp.inv_box[2]);
-  // loops over the stencil (compile-time indices into the weights), the
-  // points outside the brick skipped
+  // the weights and their derivatives are at most 1; false where the
+  // position or the cotangent is not finite
+  const bool small = fabsf(cx) + fabsf(cy) + fabsf(cz) < 1024.0f && w[0] + w[1] + w[2] <= 3.0f;
+  // loops over the stencil's x planes of this thread (compile-time indices
+  // into the weights), the points outside the brick skipped
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
-    int gx = f[0] + i;
+  for (int ii = 0; ii < N / SP; ++ii) {
+    int gx = f[0] + ii * SP + half;
     if (gx >= K0) gx -= K0;
     const int tx = gx - bx0;
     if (tx < 0 || tx >= BX) continue;
-    const float mx = M[0][i], dmx = dM[0][i];
+    float mx = M[0][ii * SP], dmx = dM[0][ii * SP];
+#pragma unroll
+    for (int h = 1; h < SP; ++h)
+      if (h == half) {
+        mx = M[0][ii * SP + h];
+        dmx = dM[0][ii * SP + h];
+      }
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       int gy = f[1] + j;
@@ -754,8 +764,8 @@ __device__ __forceinline__ void spread_dipole_atom(double4 pq, float4 c, const P
       for (int k = 0; k < N; ++k) {
         int z = f[2] + k;
         if (z >= K2) z -= K2;
-        const long long v = __double2ll_rn((double)(P * M[2][k] + Qz * dM[2][k]) * kGridScale);
-        atomicAdd(row + z, (unsigned long long)v);
+        const float v = P * M[2][k] + Qz * dM[2][k];
+        atomicAdd(row + z, small ? grid_word<true>(v) : grid_word<false>(v));
       }
     }
   }
@@ -763,8 +773,8 @@ __device__ __forceinline__ void spread_dipole_atom(double4 pq, float4 c, const P
 
 // The dipole grid of the cotangent, spread by the bricks of pme_bin's lists
 // and transformed along z like pme_spread_rows.
-template <int N, int TL>
-__global__ void __launch_bounds__(256) pme_spread_dipole(
+template <int N, int TL, int SP>
+__global__ void __launch_bounds__(SP * kBrickThreads) pme_spread_dipole(
     const double4 *__restrict__ xpq, const float4 *__restrict__ cot, PmeParams pp,
     BrickParams bp, cpx<float> *__restrict__ out, FftAxis az, size_t fs) {
   constexpr int R = BrickShape<TL>::R, BX = BrickShape<TL>::BX, BY = BrickShape<TL>::BY;
@@ -788,9 +798,9 @@ __global__ void __launch_bounds__(256) pme_spread_dipole(
   nat = nat < bp.cap ? nat : bp.cap;
   const int *lst = bp.list + (size_t)brick * bp.cap;
   __syncthreads();
-  for (int i = threadIdx.x; i < nat; i += blockDim.x) {
+  for (int i = threadIdx.x / SP; i < nat; i += blockDim.x / SP) {
     const int pl = lst[i];
-    spread_dipole_atom<N, BX, BY>(xpq[pl], cot[pl], pp, bx0, by0, acc);
+    spread_dipole_atom<N, BX, BY, SP>(xpq[pl], cot[pl], threadIdx.x % SP, pp, bx0, by0, acc);
   }
   __syncthreads();
   brick_forward_z<TL>(acc, a, b, tw, az, pp, bp, bx0, by0, out);
@@ -802,9 +812,9 @@ __global__ void __launch_bounds__(256) pme_spread_dipole(
 //   theta:   dq += c . grad phi + gs phi + psi        (word 0)
 //   Hessian: (H v)_a += q [sum_b (hess phi)_ab c_b + (grad psi)_a]
 // (gradients in x: grid-unit derivatives times K_a / L_a).
-template <int N, int TL, int BX, int BY, int KIND>
-__device__ __forceinline__ void gather_adj_atom(double4 pq, float4 c, float gs, int place,
-                                                const PmeParams &pp, int bx0, int by0,
+template <int N, int TL, int BX, int BY, int SP, int KIND>
+__device__ __forceinline__ void gather_adj_atom(double4 pq, float4 c, float gs, int half,
+                                                int place, const PmeParams &pp, int bx0, int by0,
                                                 const cpx<float> *phi, const cpx<float> *psi,
                                                 long long *__restrict__ A) {
   const int K0 = pp.K[0], K1 = pp.K[1], K2 = pp.K[2];
@@ -819,82 +829,94 @@ __device__ __forceinline__ void gather_adj_atom(double4 pq, float4 c, float gs, 
     bspline<float>(w[d], N, M[d], dM[d]);
     if (KIND == kAdjHessian) bspline_d2<N>(w[d], d2M[d]);
   }
-  // theta: phi value, grad; psi value.  Hessian: phi hessian, psi grad.
-  float v0 = 0.0f, g0 = 0.0f, g1 = 0.0f, g2 = 0.0f, p0 = 0.0f;
-  float hxx = 0.0f, hyy = 0.0f, hzz = 0.0f, hxy = 0.0f, hxz = 0.0f, hyz = 0.0f;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    int gx = f[0] + i;
-    if (gx >= K0) gx -= K0;
-    const int tx = gx - bx0;
-    if (tx < 0 || tx >= BX) continue;
-    const float mx = M[0][i], dmx = dM[0][i];
-    const float d2x = KIND == kAdjHessian ? d2M[0][i] : 0.0f;
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      int gy = f[1] + j;
-      if (gy >= K1) gy -= K1;
-      const int ty = gy - by0;
-      if (ty < 0 || ty >= BY) continue;
-      const float my = M[1][j], dmy = dM[1][j];
-      const float d2y = KIND == kAdjHessian ? d2M[1][j] : 0.0f;
-      const int r = tx * BY + ty;
-      float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, q0 = 0.0f, q1 = 0.0f;
-#pragma unroll
-      for (int k = 0; k < N; ++k) {
-        int z = f[2] + k;
-        if (z >= K2) z -= K2;
-        const cpx<float> cp = phi[z * TL + (r >> 1)];
-        const cpx<float> cs = psi[z * TL + (r >> 1)];
-        const float pv = (r & 1) ? cp.y : cp.x;
-        const float sv = (r & 1) ? cs.y : cs.x;
-        s0 += pv * M[2][k];
-        s1 += pv * dM[2][k];
-        q0 += sv * M[2][k];
-        if (KIND == kAdjHessian) {
-          s2 += pv * d2M[2][k];
-          q1 += sv * dM[2][k];
-        }
-      }
-      if (KIND == kAdjTheta) {
-        v0 += mx * my * s0;
-        g0 += dmx * my * s0;
-        g1 += mx * dmy * s0;
-        g2 += mx * my * s1;
-        p0 += mx * my * q0;
-      } else {
-        hxx += d2x * my * s0;
-        hyy += mx * d2y * s0;
-        hzz += mx * my * s2;
-        hxy += dmx * dmy * s0;
-        hxz += dmx * my * s1;
-        hyz += mx * dmy * s1;
-        g0 += dmx * my * q0;
-        g1 += mx * dmy * q0;
-        g2 += mx * my * q1;
-      }
-    }
-  }
   const float sx = (float)(K0 * pp.inv_box[0]), sy = (float)(K1 * pp.inv_box[1]),
               sz = (float)(K2 * pp.inv_box[2]);
-  unsigned long long *u = reinterpret_cast<unsigned long long *>(A + 3 * place);
-  if (KIND == kAdjTheta) {
-    const float dq = c.x * sx * g0 + c.y * sy * g1 + c.z * sz * g2 + gs * v0 + p0;
-    atomicAdd(u, (unsigned long long)to_fixed_adj(dq));
-  } else {
-    const float q = (float)pq.w;
-    const float cx = c.x * sx, cy = c.y * sy, cz = c.z * sz;
-    const float ox = q * sx * (hxx * cx + hxy * cy + hxz * cz + g0);
-    const float oy = q * sy * (hxy * cx + hyy * cy + hyz * cz + g1);
-    const float oz = q * sz * (hxz * cx + hyz * cy + hzz * cz + g2);
-    atomicAdd(u + 0, (unsigned long long)to_fixed_adj(ox));
-    atomicAdd(u + 1, (unsigned long long)to_fixed_adj(oy));
-    atomicAdd(u + 2, (unsigned long long)to_fixed_adj(oz));
+  const float q = (float)pq.w, cx = c.x * sx, cy = c.y * sy, cz = c.z * sz;
+  // the even and the odd x planes are summed apart and added as words, so
+  // that one thread and two give the same bits
+  long long wd[3] = {0, 0, 0};
+#pragma unroll
+  for (int h = 0; h < 2 / SP; ++h) {
+    const int par = SP == 2 ? half : h;
+    // theta: phi value, grad; psi value.  Hessian: phi hessian, psi grad.
+    float v0 = 0.0f, g0 = 0.0f, g1 = 0.0f, g2 = 0.0f, p0 = 0.0f;
+    float hxx = 0.0f, hyy = 0.0f, hzz = 0.0f, hxy = 0.0f, hxz = 0.0f, hyz = 0.0f;
+#pragma unroll
+    for (int ii = 0; ii < N / 2; ++ii) {
+      int gx = f[0] + 2 * ii + par;
+      if (gx >= K0) gx -= K0;
+      const int tx = gx - bx0;
+      if (tx < 0 || tx >= BX) continue;
+      const float mx = par ? M[0][2 * ii + 1] : M[0][2 * ii];
+      const float dmx = par ? dM[0][2 * ii + 1] : dM[0][2 * ii];
+      float d2x = 0.0f;
+      if (KIND == kAdjHessian) d2x = par ? d2M[0][2 * ii + 1] : d2M[0][2 * ii];
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        int gy = f[1] + j;
+        if (gy >= K1) gy -= K1;
+        const int ty = gy - by0;
+        if (ty < 0 || ty >= BY) continue;
+        const float my = M[1][j], dmy = dM[1][j];
+        const float d2y = KIND == kAdjHessian ? d2M[1][j] : 0.0f;
+        const int r = tx * BY + ty;
+        float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, q0 = 0.0f, q1 = 0.0f;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+          int z = f[2] + k;
+          if (z >= K2) z -= K2;
+          const cpx<float> cp = phi[z * TL + (r >> 1)];
+          const cpx<float> cs = psi[z * TL + (r >> 1)];
+          const float pv = (r & 1) ? cp.y : cp.x;
+          const float sv = (r & 1) ? cs.y : cs.x;
+          s0 += pv * M[2][k];
+          s1 += pv * dM[2][k];
+          q0 += sv * M[2][k];
+          if (KIND == kAdjHessian) {
+            s2 += pv * d2M[2][k];
+            q1 += sv * dM[2][k];
+          }
+        }
+        if (KIND == kAdjTheta) {
+          v0 += mx * my * s0;
+          g0 += dmx * my * s0;
+          g1 += mx * dmy * s0;
+          g2 += mx * my * s1;
+          p0 += mx * my * q0;
+        } else {
+          hxx += d2x * my * s0;
+          hyy += mx * d2y * s0;
+          hzz += mx * my * s2;
+          hxy += dmx * dmy * s0;
+          hxz += dmx * my * s1;
+          hyz += mx * dmy * s1;
+          g0 += dmx * my * q0;
+          g1 += mx * dmy * q0;
+          g2 += mx * my * q1;
+        }
+      }
+    }
+    if (KIND == kAdjTheta) {
+      wd[0] += to_fixed_adj(c.x * sx * g0 + c.y * sy * g1 + c.z * sz * g2 + gs * v0 + p0);
+    } else {
+      wd[0] += to_fixed_adj(q * sx * (hxx * cx + hxy * cy + hxz * cz + g0));
+      wd[1] += to_fixed_adj(q * sy * (hxy * cx + hyy * cy + hyz * cz + g1));
+      wd[2] += to_fixed_adj(q * sz * (hxz * cx + hyz * cy + hzz * cz + g2));
+    }
   }
+  constexpr int words = KIND == kAdjTheta ? 1 : 3;
+  if (SP == 2) {
+#pragma unroll
+    for (int k = 0; k < words; ++k) wd[k] += __shfl_xor(wd[k], 1);
+    if (half) return;
+  }
+  unsigned long long *u = reinterpret_cast<unsigned long long *>(A + 3 * (size_t)place);
+#pragma unroll
+  for (int k = 0; k < words; ++k) atomicAdd(u + k, (unsigned long long)wd[k]);
 }
 
-template <int N, int TL, int KIND>
-__global__ void __launch_bounds__(256) pme_gather_adj(
+template <int N, int TL, int SP, int KIND>
+__global__ void __launch_bounds__(SP * kBrickThreads) pme_gather_adj(
     const double4 *__restrict__ xpq, const float4 *__restrict__ cot,
     const double *__restrict__ meta, PmeParams pp, BrickParams bp,
     const cpx<float> *__restrict__ in_phi, const cpx<float> *__restrict__ in_psi, FftAxis az,
@@ -927,9 +949,10 @@ __global__ void __launch_bounds__(256) pme_gather_adj(
   __syncthreads();
   const cpx<float> *psi = brick_backward_z<TL>(in_psi, a2, b2, tw, az, pp, bp, bx0, by0);
   __syncthreads();
-  for (int i = threadIdx.x; i < nat; i += blockDim.x) {
+  for (int i = threadIdx.x / SP; i < nat; i += blockDim.x / SP) {
     const int pl = lst[i];
-    gather_adj_atom<N, TL, BX, BY, KIND>(xpq[pl], cot[pl], gs, pl, pp, bx0, by0, phi, psi, A);
+    gather_adj_atom<N, TL, BX, BY, SP, KIND>(xpq[pl], cot[pl], gs, threadIdx.x % SP, pl, pp,
+                                             bx0, by0, phi, psi, A);
   }
   __syncthreads();  // every thread has read the count
   if (threadIdx.x == 0) bp.count[brick] = 0;

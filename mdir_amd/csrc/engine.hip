@@ -1331,6 +1331,16 @@ struct Engine {
     bp.plane_major = plane_fft() ? 1 : 0;
   }
 
+  // Two threads to a listed atom (SP = 2) while the GPU holds the launch's
+  // blocks at once, four to a CU.  Alone, spread and gather: 16.2 and 16.4
+  // before, 13.5 and 16.8 with SP = 1, 11.8 and 15.3 us with SP = 2 at 256
+  // blocks (24,000 atoms); 50 steps of 14,000 atoms at order 6 (126 blocks)
+  // 4,487, 4,522, 4,317 us.  At 2,916 blocks (999,000 atoms) the spread
+  // alone is faster still (176, 142, 115 us), but the larger blocks wait for
+  // room beside the pair loop: a pass of 114.0, 112.7, 124.0 ms; 64 frames
+  // (4,096 blocks) 925, 922, 1,016 us.
+  static constexpr int kSplitBlocks = 1024;
+  int brick_split() const { return nbricks * nz <= kSplitBlocks ? 2 : 1; }
   const double4 *pme_positions() const { return pme_atoms ? d_xpa : d_xpq; }
 
   // Lists the atoms of every brick their stencils touch.
@@ -1360,7 +1370,9 @@ struct Engine {
     static_assert(BX * BY == R, "brick shape");
     const int blocks = ((pme_grid[0] + BX - 1) / BX) * ((pme_grid[1] + BY - 1) / BY);
     const size_t lds = (size_t)(32 * TL + 8) * pme_grid[2];
-    pme_spread_rows<N, TL><<<dim3(blocks, 1, nz), 256, lds, pstream>>>(
+    const int sp = brick_split();
+    const auto kernel = sp == 2 ? pme_spread_rows<N, TL, 2> : pme_spread_rows<N, TL, 1>;
+    kernel<<<dim3(blocks, 1, nz), sp * kBrickThreads, lds, pstream>>>(
         pme_positions(), pmp, bp, d_cplx, fft.ax[2].axis, fs);
   }
   template <int N>
@@ -1377,7 +1389,9 @@ struct Engine {
     constexpr int BX = BrickShape<TL>::BX, BY = BrickShape<TL>::BY;
     const int blocks = ((pme_grid[0] + BX - 1) / BX) * ((pme_grid[1] + BY - 1) / BY);
     const size_t lds = (size_t)(16 * TL + 8) * pme_grid[2];
-    pme_gather_rows<N, TL><<<dim3(blocks, 1, nz), 256, lds, pstream>>>(
+    const int sp = brick_split();
+    const auto kernel = sp == 2 ? pme_gather_rows<N, TL, 2> : pme_gather_rows<N, TL, 1>;
+    kernel<<<dim3(blocks, 1, nz), sp * kBrickThreads, lds, pstream>>>(
         pme_positions(), pmp, bp, d_cplx, fft.ax[2].axis, pme_atoms ? d_Fr : d_F, fs);
   }
   template <int N>

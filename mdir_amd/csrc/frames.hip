@@ -428,10 +428,14 @@ struct FrameBatch {
     static_assert(BX * BY == R, "brick shape");
     const int blocks = ((e.pme_grid[0] + BX - 1) / BX) * ((e.pme_grid[1] + BY - 1) / BY);
     const size_t lds = (size_t)(32 * TL + 8) * e.pme_grid[2];
-    pme_spread_dipole<N, TL><<<dim3(blocks, 1, e.nz), 256, lds, e.pstream>>>(
+    const int sp = e.brick_split(), threads = sp * kBrickThreads;
+    const auto spread = sp == 2 ? pme_spread_dipole<N, TL, 2> : pme_spread_dipole<N, TL, 1>;
+    const auto gather =
+        sp == 2 ? pme_gather_adj<N, TL, 2, KIND> : pme_gather_adj<N, TL, 1, KIND>;
+    spread<<<dim3(blocks, 1, e.nz), threads, lds, e.pstream>>>(
         e.d_xpq, d_cot, e.pmp, e.bp, d_cplx2, e.fft.ax[2].axis, e.fs);
     e.plane_conv(d_cplx2, nullptr, nullptr);
-    pme_gather_adj<N, TL, KIND><<<dim3(blocks, 1, e.nz), 256, lds, e.pstream>>>(
+    gather<<<dim3(blocks, 1, e.nz), threads, lds, e.pstream>>>(
         e.d_xpq, d_cot, d_meta, e.pmp, e.bp, e.d_cplx, d_cplx2, e.fft.ax[2].axis, d_A, e.fs);
   }
   template <int N, int KIND>

@@ -107,21 +107,15 @@ template <int TL> struct BrickShape {
   static constexpr int BX = R / BY;
 };
 
-// The bricks along one axis that the stencil f, f+1, .., f+N-1 (mod K)
-// touches, each once.
+// The bricks along one axis, nb of B points each (the last one may hold
+// fewer of the K), that the stencil f .. f+N-1 (mod K) touches: `count`
+// bricks from `first` on, mod nb.  A stencil of at most K/2 points never
+// comes back to its first brick.
 template <int N, int B>
-__device__ __forceinline__ int stencil_bricks(int f, int K, int *out) {
-  int n = 0;
-#pragma unroll
-  for (int k = 0; k < N; ++k) {
-    int p = f + k;
-    if (p >= K) p -= K;
-    const int b = p / B;
-    bool seen = false;
-    for (int j = 0; j < n; ++j) seen |= out[j] == b;
-    if (!seen) out[n++] = b;
-  }
-  return n;
+__device__ __forceinline__ void stencil_bricks(int f, int K, int nb, int &first, int &count) {
+  const int l = f + N - 1;
+  first = f / B;
+  count = l < K ? l / B - first + 1 : nb - first + (l - K) / B + 1;
 }
 
 // Thread per place: list the place with every brick its stencil touches.
@@ -147,7 +141,11 @@ __global__ void __launch_bounds__(256) pme_bin(const int *__restrict__ counts,
   if (lds)
     for (int k = threadIdx.x; k < nbricks; k += blockDim.x) s_count[k] = 0;
   const int place = blockIdx.x * blockDim.x + threadIdx.x;
-  int bx[N], by[N], nx = 0, ny = 0;
+  // at most this many bricks per axis: whole ones, one more at each end, a
+  // partial one at the wrap
+  constexpr int MX = (N - 2) / BX + 3 < N ? (N - 2) / BX + 3 : N;
+  constexpr int MY = (N - 2) / BY + 3 < N ? (N - 2) / BY + 3 : N;
+  int bx = 0, by = 0, nx = 0, ny = 0;
   if (place < counts[0]) {
     const double4 pq = xpq[place];
     if (pq.w != 0.0) {  // not padding, not an uncharged atom
@@ -155,15 +153,23 @@ __global__ void __launch_bounds__(256) pme_bin(const int *__restrict__ counts,
       float w;
       pme_place(pq.x, pp.box[0], pp.inv_box[0], pp.K[0], N, f0, w);
       pme_place(pq.y, pp.box[1], pp.inv_box[1], pp.K[1], N, f1, w);
-      nx = stencil_bricks<N, BX>(f0, pp.K[0], bx);
-      ny = stencil_bricks<N, BY>(f1, pp.K[1], by);
+      stencil_bricks<N, BX>(f0, pp.K[0], bp.nbx, bx, nx);
+      stencil_bricks<N, BY>(f1, pp.K[1], bp.nby, by, ny);
     }
   }
-  int local[N * N];
+  auto brick_at = [&](int i, int j) {
+    const int x = bx + i, y = by + j;
+    return (y < bp.nby ? y : y - bp.nby) * bp.nbx + (x < bp.nbx ? x : x - bp.nbx);
+  };
+  // unrolled to the most bricks, so that `local` stays in registers
+  int local[MX * MY];
   if (lds) {
     __syncthreads();
-    for (int j = 0; j < ny; ++j)
-      for (int i = 0; i < nx; ++i) local[j * N + i] = atomicAdd(&s_count[by[j] * bp.nbx + bx[i]], 1);
+#pragma unroll
+    for (int j = 0; j < MY; ++j)
+#pragma unroll
+      for (int i = 0; i < MX; ++i)
+        if (i < nx && j < ny) local[j * MX + i] = atomicAdd(&s_count[brick_at(i, j)], 1);
     __syncthreads();
     for (int k = threadIdx.x; k < nbricks; k += blockDim.x) {
       const int c = s_count[k];
@@ -171,10 +177,13 @@ __global__ void __launch_bounds__(256) pme_bin(const int *__restrict__ counts,
     }
     __syncthreads();
   }
-  for (int j = 0; j < ny; ++j)
-    for (int i = 0; i < nx; ++i) {
-      const int brick = by[j] * bp.nbx + bx[i];
-      const int slot = lds ? s_count[brick] + local[j * N + i] : atomicAdd(&bp.count[brick], 1);
+#pragma unroll
+  for (int j = 0; j < MY; ++j)
+#pragma unroll
+    for (int i = 0; i < MX; ++i) {
+      if (i >= nx || j >= ny) continue;
+      const int brick = brick_at(i, j);
+      const int slot = lds ? s_count[brick] + local[j * MX + i] : atomicAdd(&bp.count[brick], 1);
       if (slot < bp.cap)
         bp.list[(size_t)brick * bp.cap + slot] = place;
       else
@@ -182,52 +191,84 @@ __global__ void __launch_bounds__(256) pme_bin(const int *__restrict__ counts,
     }
 }
 
-// The part of one atom's stencil (place-ordered position and charge pq)
-// that lies in the brick at (bx0, by0), added to the brick's accumulators.
-template <int N, int BX, int BY>
-__device__ __forceinline__ void spread_atom(double4 pq, const PmeParams &pp, int bx0,
-                                            int by0, unsigned long long *acc) {
+// The spread, the gather and their adjoints come with SP = 1 and SP = 2
+// threads to a listed atom, each taking every SP-th x plane of its stencil,
+// in blocks of SP kBrickThreads.  A brick lists a few hundred atoms: while
+// the GPU holds all blocks at once, what a block waits for is the serial
+// chain of one atom's stencil and of its own rows' transform, and two
+// threads halve both; beyond that the second thread's own weights, and
+// blocks twice as large to find room for beside the pair loop, cost more.
+constexpr int kBrickThreads = 256;
+
+// The word nearest p 2^40, ties to even, as __double2ll_rn(p 2^40) gives
+// it, for |p| < 2^11: the sum with 1.5 2^52 is rounded at its last bit, a
+// unit, and holds the integer in its mantissa: two f64 operations instead
+// of eight.
+__device__ __forceinline__ unsigned long long grid_word_small(float p) {
+  const double d = fma((double)p, kGridScale, 0x1.8p52);
+  return (unsigned long long)(__double_as_longlong(d) - 0x4338000000000000ll);
+}
+template <bool SMALL>
+__device__ __forceinline__ unsigned long long grid_word(float p) {
+  if (SMALL) return grid_word_small(p);
+  return (unsigned long long)__double2ll_rn((double)p * kGridScale);
+}
+
+// The x planes `half`, half + SP, .. of one atom's stencil (first
+// points f, weights M, charge q), the part that lies in the brick at (bx0,
+// by0), added to the brick's accumulators.  SMALL: every product is below
+// 2^11.
+template <int N, int BX, int BY, int SP, bool SMALL>
+__device__ __forceinline__ void spread_part(const int (&f)[3], const float (&M)[3][N], float qf,
+                                            int half, const PmeParams &pp, int bx0, int by0,
+                                            unsigned long long *acc) {
   const int K0 = pp.K[0], K1 = pp.K[1], K2 = pp.K[2];
-  const double qd = pq.w;
+  int z[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) z[k] = f[2] + k < K2 ? f[2] + k : f[2] + k - K2;
+#pragma unroll
+  for (int ii = 0; ii < N / SP; ++ii) {
+    int gx = f[0] + ii * SP + half;
+    if (gx >= K0) gx -= K0;
+    const int tx = gx - bx0;
+    if (tx < 0 || tx >= BX) continue;
+    float mx = M[0][ii * SP];
+#pragma unroll
+    for (int h = 1; h < SP; ++h)
+      if (h == half) mx = M[0][ii * SP + h];
+    const float wx = mx * qf;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      int gy = f[1] + j;
+      if (gy >= K1) gy -= K1;
+      const int ty = gy - by0;
+      if (ty < 0 || ty >= BY) continue;
+      const float wxy = M[1][j] * wx;
+      unsigned long long *row = acc + (tx * BY + ty) * K2;
+#pragma unroll
+      for (int k = 0; k < N; ++k) atomicAdd(row + z[k], grid_word<SMALL>(wxy * M[2][k]));
+    }
+  }
+}
+
+template <int N, int BX, int BY, int SP>
+__device__ __forceinline__ void spread_atom(double4 pq, int half, const PmeParams &pp, int bx0,
+                                            int by0, unsigned long long *acc) {
   int f[3];
   float w[3];
-  pme_place(pq.x, pp.box[0], pp.inv_box[0], K0, N, f[0], w[0]);
-  pme_place(pq.y, pp.box[1], pp.inv_box[1], K1, N, f[1], w[1]);
-  pme_place(pq.z, pp.box[2], pp.inv_box[2], K2, N, f[2], w[2]);
+  pme_place(pq.x, pp.box[0], pp.inv_box[0], pp.K[0], N, f[0], w[0]);
+  pme_place(pq.y, pp.box[1], pp.inv_box[1], pp.K[1], N, f[1], w[1]);
+  pme_place(pq.z, pp.box[2], pp.inv_box[2], pp.K[2], N, f[2], w[2]);
   float M[3][N];
 #pragma unroll
   for (int d = 0; d < 3; ++d) bspline<float>(w[d], N, M[d], nullptr);
-  const float qf = (float)qd;
-#pragma unroll
-  for (int tx = 0; tx < BX; ++tx) {
-    int kx = bx0 + tx - f[0];
-    if (kx < 0) kx += K0;
-    if (kx >= N || bx0 + tx >= K0) continue;
-    float wx = M[0][0];
-#pragma unroll
-    for (int k = 1; k < N; ++k)
-      if (k == kx) wx = M[0][k];
-    wx *= qf;
-#pragma unroll
-    for (int ty = 0; ty < BY; ++ty) {
-      int ky = by0 + ty - f[1];
-      if (ky < 0) ky += K1;
-      if (ky >= N || by0 + ty >= K1) continue;
-      float wxy = M[1][0];
-#pragma unroll
-      for (int k = 1; k < N; ++k)
-        if (k == ky) wxy = M[1][k];
-      wxy *= wx;
-      unsigned long long *row = acc + (tx * BY + ty) * K2;
-#pragma unroll
-      for (int k = 0; k < N; ++k) {
-        int z = f[2] + k;
-        if (z >= K2) z -= K2;
-        const long long v = __double2ll_rn((double)(wxy * M[2][k]) * kGridScale);
-        atomicAdd(row + z, (unsigned long long)v);
-      }
-    }
-  }
+  const float qf = (float)pq.w;
+  // the weights are at most 1; the second test is false for a position
+  // that is not finite
+  if (fabsf(qf) < 1024.0f && w[0] + w[1] + w[2] <= 3.0f)
+    spread_part<N, BX, BY, SP, true>(f, M, qf, half, pp, bx0, by0, acc);
+  else
+    spread_part<N, BX, BY, SP, false>(f, M, qf, half, pp, bx0, by0, acc);
 }
 
 // The brick's R accumulated real rows (64-bit words in acc) to their half
@@ -274,8 +315,8 @@ __device__ __forceinline__ void brick_forward_z(const unsigned long long *acc,
   }
 }
 
-template <int N, int TL>
-__global__ void __launch_bounds__(256) pme_spread_rows(
+template <int N, int TL, int SP>
+__global__ void __launch_bounds__(SP * kBrickThreads) pme_spread_rows(
     const double4 *__restrict__ xpq, PmeParams pp, BrickParams bp,
     cpx<float> *__restrict__ out, FftAxis az, size_t fs) {
   constexpr int R = BrickShape<TL>::R, BX = BrickShape<TL>::BX, BY = BrickShape<TL>::BY;
@@ -298,13 +339,15 @@ __global__ void __launch_bounds__(256) pme_spread_rows(
   nat = nat < bp.cap ? nat : bp.cap;
   const int *lst = bp.list + (size_t)brick * bp.cap;
   __syncthreads();
-  // two atoms per thread in flight: their loads are independent
-  for (int i0 = threadIdx.x; i0 < nat; i0 += 2 * blockDim.x) {
-    const int i1 = i0 + blockDim.x;
-    const double4 a0 = xpq[lst[i0]];
-    const double4 a1 = i1 < nat ? xpq[lst[i1]] : make_double4(0, 0, 0, 0);
-    spread_atom<N, BX, BY>(a0, pp, bx0, by0, acc);
-    if (i1 < nat) spread_atom<N, BX, BY>(a1, pp, bx0, by0, acc);
+  // the next atom's load is in flight while this one is spread
+  const int half = threadIdx.x % SP, step = blockDim.x / SP;
+  int i = threadIdx.x / SP;
+  double4 pq = i < nat ? xpq[lst[i]] : make_double4(0, 0, 0, 0);
+  while (i < nat) {
+    i += step;
+    const double4 next = i < nat ? xpq[lst[i]] : make_double4(0, 0, 0, 0);
+    spread_atom<N, BX, BY, SP>(pq, half, pp, bx0, by0, acc);
+    pq = next;
   }
   __syncthreads();
   brick_forward_z<TL>(acc, a, b, tw, az, pp, bp, bx0, by0, out);
@@ -320,15 +363,15 @@ __global__ void __launch_bounds__(256) pme_spread_rows(
 // HBM.  The block clears its brick's list count for the next step.
 
 // One atom's force from the potential rows of the brick at (bx0, by0):
-// -q (K/L) sum phi M' M M over the stencil points in the brick, added as
+// -q (K/L) sum phi M' M M over the stencil points in the brick, summed over
+// the SP neighbouring threads that share the atom and added as
 // 64-bit fixed point.  phi of brick row r at z is phi[z TL + r/2], .x for
 // even r and .y for odd r.
-template <int N, int TL, int BX, int BY>
-__device__ __forceinline__ void gather_atom(double4 pq, int place, const PmeParams &pp,
+template <int N, int TL, int BX, int BY, int SP>
+__device__ __forceinline__ void gather_atom(double4 pq, int half, int place, const PmeParams &pp,
                                             int bx0, int by0, const cpx<float> *phi,
                                             long long *__restrict__ F) {
   const int K0 = pp.K[0], K1 = pp.K[1], K2 = pp.K[2];
-  const double qd = pq.w;
   int f[3];
   float w[3];
   pme_place(pq.x, pp.box[0], pp.inv_box[0], K0, N, f[0], w[0]);
@@ -337,52 +380,62 @@ __device__ __forceinline__ void gather_atom(double4 pq, int place, const PmePara
   float M[3][N], dM[3][N];
 #pragma unroll
   for (int d = 0; d < 3; ++d) bspline<float>(w[d], N, M[d], dM[d]);
-  float g0 = 0.0f, g1 = 0.0f, g2 = 0.0f;
+  const float *flat = reinterpret_cast<const float *>(phi);
+  int z[N];
 #pragma unroll
-  for (int tx = 0; tx < BX; ++tx) {
-    int kx = bx0 + tx - f[0];
-    if (kx < 0) kx += K0;
-    if (kx >= N || bx0 + tx >= K0) continue;
-    float mx = M[0][0], dmx = dM[0][0];
+  for (int k = 0; k < N; ++k) z[k] = 2 * TL * (f[2] + k < K2 ? f[2] + k : f[2] + k - K2);
+  const float qf = (float)pq.w;
+  const float s0 = -qf * (float)(K0 * pp.inv_box[0]), s1 = -qf * (float)(K1 * pp.inv_box[1]),
+              s2 = -qf * (float)(K2 * pp.inv_box[2]);
+  // the even and the odd x planes are summed apart and added as words, so
+  // that one thread and two give the same bits
+  long long w0 = 0, w1 = 0, w2 = 0;
 #pragma unroll
-    for (int k = 1; k < N; ++k)
-      if (k == kx) {
-        mx = M[0][k];
-        dmx = dM[0][k];
-      }
+  for (int h = 0; h < 2 / SP; ++h) {
+    const int par = SP == 2 ? half : h;
+    float g0 = 0.0f, g1 = 0.0f, g2 = 0.0f;
 #pragma unroll
-    for (int ty = 0; ty < BY; ++ty) {
-      int ky = by0 + ty - f[1];
-      if (ky < 0) ky += K1;
-      if (ky >= N || by0 + ty >= K1) continue;
-      float my = M[1][0], dmy = dM[1][0];
+    for (int ii = 0; ii < N / 2; ++ii) {
+      int gx = f[0] + 2 * ii + par;
+      if (gx >= K0) gx -= K0;
+      const int tx = gx - bx0;
+      if (tx < 0 || tx >= BX) continue;
+      const float mx = par ? M[0][2 * ii + 1] : M[0][2 * ii];
+      const float dmx = par ? dM[0][2 * ii + 1] : dM[0][2 * ii];
 #pragma unroll
-      for (int k = 1; k < N; ++k)
-        if (k == ky) {
-          my = M[1][k];
-          dmy = dM[1][k];
+      for (int j = 0; j < N; ++j) {
+        int gy = f[1] + j;
+        if (gy >= K1) gy -= K1;
+        const int ty = gy - by0;
+        if (ty < 0 || ty >= BY) continue;
+        const float my = M[1][j], dmy = dM[1][j];
+        const float *row = flat + tx * BY + ty;
+        float sz = 0.0f, dsz = 0.0f;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+          const float pv = row[z[k]];
+          sz += pv * M[2][k];
+          dsz += pv * dM[2][k];
         }
-      const int r = tx * BY + ty;
-      float sz = 0.0f, dsz = 0.0f;
-#pragma unroll
-      for (int k = 0; k < N; ++k) {
-        int z = f[2] + k;
-        if (z >= K2) z -= K2;
-        const cpx<float> c = phi[z * TL + (r >> 1)];
-        const float pv = (r & 1) ? c.y : c.x;
-        sz += pv * M[2][k];
-        dsz += pv * dM[2][k];
+        g0 += dmx * my * sz;
+        g1 += mx * dmy * sz;
+        g2 += mx * my * dsz;
       }
-      g0 += dmx * my * sz;
-      g1 += mx * dmy * sz;
-      g2 += mx * my * dsz;
     }
+    w0 += to_fixed(s0 * g0);
+    w1 += to_fixed(s1 * g1);
+    w2 += to_fixed(s2 * g2);
   }
-  const float qf = (float)qd;
-  unsigned long long *u = reinterpret_cast<unsigned long long *>(F + 3 * place);
-  atomicAdd(u + 0, (unsigned long long)to_fixed(-qf * (float)(K0 * pp.inv_box[0]) * g0));
-  atomicAdd(u + 1, (unsigned long long)to_fixed(-qf * (float)(K1 * pp.inv_box[1]) * g1));
-  atomicAdd(u + 2, (unsigned long long)to_fixed(-qf * (float)(K2 * pp.inv_box[2]) * g2));
+  if (SP == 2) {
+    w0 += __shfl_xor(w0, 1);
+    w1 += __shfl_xor(w1, 1);
+    w2 += __shfl_xor(w2, 1);
+    if (half) return;
+  }
+  unsigned long long *u = reinterpret_cast<unsigned long long *>(F + 3 * (size_t)place);
+  atomicAdd(u + 0, (unsigned long long)w0);
+  atomicAdd(u + 1, (unsigned long long)w1);
+  atomicAdd(u + 2, (unsigned long long)w2);
 }
 
 // The brick's half-spectrum rows of `in` back to real rows in LDS (one
@@ -422,8 +475,8 @@ __device__ __forceinline__ const cpx<float> *brick_backward_z(
   return lds_fft<float, TL, 1>(a, b, az, tw);
 }
 
-template <int N, int TL>
-__global__ void __launch_bounds__(256) pme_gather_rows(
+template <int N, int TL, int SP>
+__global__ void __launch_bounds__(SP * kBrickThreads) pme_gather_rows(
     const double4 *__restrict__ xpq, PmeParams pp, BrickParams bp,
     const cpx<float> *__restrict__ in, FftAxis az, long long *__restrict__ F, size_t fs) {
   constexpr int BX = BrickShape<TL>::BX, BY = BrickShape<TL>::BY;
@@ -444,15 +497,19 @@ __global__ void __launch_bounds__(256) pme_gather_rows(
   int nat = bp.count[brick];
   nat = nat < bp.cap ? nat : bp.cap;
   const int *lst = bp.list + (size_t)brick * bp.cap;
+  // the first atoms load while the rows are transformed
+  const int half = threadIdx.x % SP, step = blockDim.x / SP;
+  int i = threadIdx.x / SP;
+  int place = i < nat ? lst[i] : 0;
+  double4 pq = xpq[place];
   const cpx<float> *phi = brick_backward_z<TL>(in, a, b, tw, az, pp, bp, bx0, by0);
-  for (int i0 = threadIdx.x; i0 < nat; i0 += 2 * blockDim.x) {
-    const int i1 = i0 + blockDim.x;
-    const int p0 = lst[i0];
-    const int p1 = i1 < nat ? lst[i1] : p0;
-    const double4 a0 = xpq[p0];
-    const double4 a1 = xpq[p1];
-    gather_atom<N, TL, BX, BY>(a0, p0, pp, bx0, by0, phi, F);
-    if (i1 < nat) gather_atom<N, TL, BX, BY>(a1, p1, pp, bx0, by0, phi, F);
+  while (i < nat) {
+    i += step;
+    const int next_place = i < nat ? lst[i] : 0;
+    const double4 next = xpq[next_place];
+    gather_atom<N, TL, BX, BY, SP>(pq, half, place, pp, bx0, by0, phi, F);
+    place = next_place;
+    pq = next;
   }
   __syncthreads();  // every thread has read the count
   if (threadIdx.x == 0) bp.count[brick] = 0;
@@ -805,13 +862,15 @@ __global__ void __launch_bounds__(512) fft_plane_conv(cpx<float> *__restrict__ d
 }
 
 template __global__ void fft_rows_r2c<float, true>(const void *, cpx<float> *, int, FftAxis);
+#define MDHIP_SPREAD_SP(N, TL, SP)                                                       \
+  template __global__ void pme_spread_rows<N, TL, SP>(const double4 *, PmeParams,        \
+      BrickParams, cpx<float> *, FftAxis, size_t);                                       \
+  template __global__ void pme_gather_rows<N, TL, SP>(const double4 *, PmeParams,        \
+      BrickParams, const cpx<float> *, FftAxis, long long *, size_t);
 #define MDHIP_SPREAD(N, TL)                                                              \
   template __global__ void pme_bin<N, TL>(const int *, const double4 *, PmeParams,       \
       BrickParams, int *, size_t);                                                       \
-  template __global__ void pme_spread_rows<N, TL>(const double4 *, PmeParams,            \
-      BrickParams, cpx<float> *, FftAxis, size_t);                                       \
-  template __global__ void pme_gather_rows<N, TL>(const double4 *, PmeParams,            \
-      BrickParams, const cpx<float> *, FftAxis, long long *, size_t);
+  MDHIP_SPREAD_SP(N, TL, 1) MDHIP_SPREAD_SP(N, TL, 2)
 #define MDHIP_SPREAD_N(N) MDHIP_SPREAD(N, 8) MDHIP_SPREAD(N, 4) MDHIP_SPREAD(N, 2) MDHIP_SPREAD(N, 1)
 MDHIP_SPREAD_N(4)
 MDHIP_SPREAD_N(6)
