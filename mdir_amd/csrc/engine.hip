@@ -32,6 +32,7 @@
 #include "integrate.hip"
 #include "nbnxm.hip"
 #include "bonded.hip"
+#include "sums.hip"
 #include "pairs.hip"
 #include "pme.hip"
 #include "pme_mfma.hip"
@@ -180,7 +181,7 @@ struct Engine {
 
   // ---- state (atom order) ----
   double *d_x = nullptr, *d_v = nullptr, *d_xref = nullptr, *d_shift = nullptr;
-  double *d_q = nullptr, *d_inv_mass = nullptr;
+  double *d_q = nullptr, *d_inv_mass = nullptr, *d_mass = nullptr;
   int *d_type = nullptr, *d_place_of = nullptr;
   double *d_save_x = nullptr, *d_save_v = nullptr;
 
@@ -678,7 +679,7 @@ struct Engine {
     dfree(d_timing);
     timing_slots = 0;
     dfree(d_x); dfree(d_v); dfree(d_xref); dfree(d_shift); dfree(d_q);
-    dfree(d_inv_mass); dfree(d_type); dfree(d_place_of); dfree(d_save_x); dfree(d_save_v);
+    dfree(d_inv_mass); dfree(d_mass); dfree(d_type); dfree(d_place_of); dfree(d_save_x); dfree(d_save_v);
     dfree(d_xprune); dfree(d_xpa); dfree(d_Fr); dfree(d_pme_n);
     release_list();
     dfree(d_excl_start); dfree(d_excl_atoms); dfree(d_flags); dfree(d_lj);
@@ -691,6 +692,9 @@ struct Engine {
     dfree(d_dft1); dfree(d_dft2);
     dfree(bp.count); dfree(bp.list);
     dfree(d_unit_first); dfree(d_unit_size); dfree(d_lstep);
+    dfree(d_sums); dfree(d_fout);
+    if (h_sums) hipHostFree(h_sums);
+    h_sums = nullptr;
     if (ev_fork) hipEventDestroy(ev_fork);
     if (ev_join) hipEventDestroy(ev_join);
     ev_fork = ev_join = nullptr;
@@ -848,6 +852,7 @@ struct Engine {
     std::vector<double> im(n);
     for (int i = 0; i < n; ++i) im[i] = h_mass[i] > 0 ? 1.0 / h_mass[i] : 0.0;
     d_inv_mass = dupload(im);
+    d_mass = dupload(h_mass);
     d_type = dupload(h_type);
     d_place_of = dalloc<int>(n);
     d_flags = dalloc<int>(kNumFlags);
@@ -1826,50 +1831,65 @@ struct Engine {
     outputs(F_out, E_out);
   }
 
+  // Sums on the device (sums.hip): launched into a buffer of their own,
+  // copied to pinned memory; sum_of() after the stream is synchronised.
+  double *d_sums = nullptr, *h_sums = nullptr, *d_fout = nullptr;
+  void launch_sums(SumArgs &sa) {
+    constexpr size_t words = (size_t)kSumKinds * kSumBlocks * kSumWidth;
+    if (!d_sums) d_sums = dalloc<double>(words);
+    if (!h_sums) HIPCHK(hipHostMalloc((void **)&h_sums, words * sizeof(double), 0));
+    sa.v = d_v;
+    sa.mass = d_mass;
+    energy_sums<<<dim3(kSumBlocks, kSumKinds), 256, 0, stream>>>(sa, d_sums);
+    HIPCHK(hipMemcpyAsync(h_sums, d_sums, words * sizeof(double), hipMemcpyDeviceToHost, stream));
+  }
+  double sum_of(int kind, int component) const {
+    double e = 0.0;
+    for (int b = 0; b < kSumBlocks; ++b)
+      e += h_sums[((size_t)kind * kSumBlocks + b) * kSumWidth + component];
+    return e;
+  }
+
   // Forces (atom order, f64) and energy terms of the last evaluation.
   void outputs(double *F_out, double *E_out) {
-    if (F_out) {
-      double *d_out = dalloc<double>(3 * (size_t)n);
-      forces_to_atoms<<<blocks_for(n), 256, 0, stream>>>(n, d_place_of, d_F, d_out, 0);
-      HIPCHK(hipMemcpyAsync(F_out, d_out, 3 * n * sizeof(double), hipMemcpyDeviceToHost, stream));
-      HIPCHK(hipStreamSynchronize(stream));
-      dfree(d_out);
+    SumArgs sa{};
+    if (E_out) {
+      sa.src[kSumPairs] = d_epair;   // one partial per (piece, group) wave
+      sa.width[kSumPairs] = 2;
+      sa.count[kSumPairs] = terms & 1 ? (long long)max_groups * nseg() : 0;
+      sa.src[kSumSpecial] = d_espec;
+      sa.width[kSumSpecial] = 3;
+      sa.count[kSumSpecial] = nspecial && (terms & 2) ? blocks_for(nspecial) : 0;
+      sa.src[kSumTuples] = d_etup;
+      sa.width[kSumTuples] = kTupleKinds;
+      sa.count[kSumTuples] = tuple_blocks();
+      sa.src[kSumRecip] = d_erecip;
+      sa.width[kSumRecip] = 1;
+      sa.count[kSumRecip] = use_pme && (terms & 4) ? recip_blocks() : 0;
+      sa.n = n;
+      launch_sums(sa);
     }
+    if (F_out) {
+      if (!d_fout) d_fout = dalloc<double>(3 * (size_t)n);
+      forces_to_atoms<<<blocks_for(n), 256, 0, stream>>>(n, d_place_of, d_F, d_fout, 0);
+      HIPCHK(hipMemcpyAsync(F_out, d_fout, 3 * n * sizeof(double), hipMemcpyDeviceToHost,
+                            stream));
+    }
+    HIPCHK(hipStreamSynchronize(stream));
     if (E_out) {
       for (int k = 0; k < MDRT_NUM_ENERGIES; ++k) E_out[k] = 0.0;
-      // one partial per (segment, group) wave, summed in a fixed order
-      std::vector<double> ep(2 * (size_t)max_groups * nseg());
-      to_host(ep.data(), d_epair, ep.size() * sizeof(double));
-      for (size_t w = 0; (terms & 1) && w < ep.size() / 2; ++w) {
-        E_out[MDRT_E_LJ] += ep[2 * w];
-        E_out[MDRT_E_COUL_DIRECT] += ep[2 * w + 1];
-      }
-      if (nspecial && (terms & 2)) {
-        const int nb = blocks_for(nspecial);
-        std::vector<double> es(3 * (size_t)nb);
-        to_host(es.data(), d_espec, es.size() * sizeof(double));
-        for (int b = 0; b < nb; ++b) {
-          E_out[MDRT_E_COUL_EXCL] += es[3 * b];
-          E_out[MDRT_E_LJ14] += es[3 * b + 1];
-          E_out[MDRT_E_COUL14] += es[3 * b + 2];
-        }
-      }
-      if (const int tb = tuple_blocks()) {
-        std::vector<double> et((size_t)kTupleKinds * tb);
-        to_host(et.data(), d_etup, et.size() * sizeof(double));
-        const int slot[kTupleKinds] = {MDRT_E_BONDS, MDRT_E_UREY_BRADLEY, MDRT_E_ANGLES,
-                                       MDRT_E_DIHEDRALS, MDRT_E_IMPROPERS};
-        for (int b = 0; b < tb; ++b)
-          for (int k = 0; k < kTupleKinds; ++k) E_out[slot[k]] += et[(size_t)kTupleKinds * b + k];
-      }
-      if (use_pme && (terms & 4)) {
-        std::vector<double> er(recip_blocks());
-        to_host(er.data(), d_erecip, er.size() * sizeof(double));
-        for (double e : er) E_out[MDRT_E_COUL_RECIP] += e;
-      }
+      E_out[MDRT_E_LJ] = sum_of(kSumPairs, 0);
+      E_out[MDRT_E_COUL_DIRECT] = sum_of(kSumPairs, 1);
+      E_out[MDRT_E_COUL_EXCL] = sum_of(kSumSpecial, 0);
+      E_out[MDRT_E_LJ14] = sum_of(kSumSpecial, 1);
+      E_out[MDRT_E_COUL14] = sum_of(kSumSpecial, 2);
+      const int slot[kTupleKinds] = {MDRT_E_BONDS, MDRT_E_UREY_BRADLEY, MDRT_E_ANGLES,
+                                     MDRT_E_DIHEDRALS, MDRT_E_IMPROPERS};
+      for (int k = 0; k < kTupleKinds; ++k) E_out[slot[k]] = sum_of(kSumTuples, k);
+      E_out[MDRT_E_COUL_RECIP] = sum_of(kSumRecip, 0);
       E_out[MDRT_E_COUL_SELF] = e_self;
       E_out[MDRT_E_DISP_CORR] = e_disp;
-      E_out[MDRT_E_KINETIC] = kinetic_energy();
+      E_out[MDRT_E_KINETIC] = sum_of(kSumKinetic, 0);
     }
   }
 
@@ -1939,12 +1959,11 @@ struct Engine {
   }
 
   double kinetic_energy() {
-    std::vector<double> v(3 * (size_t)n);
-    to_host(v.data(), d_v, v.size() * sizeof(double));
-    double ke = 0;
-    for (int i = 0; i < n; ++i)
-      ke += 0.5 * h_mass[i] * (v[3 * i] * v[3 * i] + v[3 * i + 1] * v[3 * i + 1] + v[3 * i + 2] * v[3 * i + 2]);
-    return ke;
+    SumArgs sa{};
+    sa.n = n;
+    launch_sums(sa);
+    HIPCHK(hipStreamSynchronize(stream));
+    return sum_of(kSumKinetic, 0);
   }
 
   // The captured sequence of `steps` steps of dt (with the pair-loop clock
