@@ -137,15 +137,14 @@ __device__ inline double tuple_force(int kind, const double *xi, const double *x
   return u;
 }
 
-// Grid-stride over the tuples; with energy partials, kTupleKinds sums per
-// block in a fixed order.
-__global__ void __launch_bounds__(256) bonded_tuples(TupleArgs ta, const double *__restrict__ x,
-                                                     const int *__restrict__ place_of,
-                                                     double bx, double by, double bz,
-                                                     long long *__restrict__ F) {
+// Block `block` of `nblocks`, 256 threads: grid-stride over the tuples, the
+// forces added at place_of[atom], or at the atom where place_of is null;
+// with energy partials, kTupleKinds sums per block in a fixed order.
+__device__ __forceinline__ void tuple_block(int block, int nblocks, const TupleArgs &ta,
+                                            const double *__restrict__ x,
+                                            const int *__restrict__ place_of,
+                                            const double *box, long long *__restrict__ F) {
   __shared__ double s_e[1][256];
-  const double box[3] = {bx, by, bz};
-  const int block = blockIdx.x, nblocks = gridDim.x;
   double e[kTupleKinds] = {0.0, 0.0, 0.0, 0.0, 0.0};
   for (int t = block * (int)blockDim.x + (int)threadIdx.x; t < ta.ntuples;
        t += nblocks * (int)blockDim.x) {
@@ -157,10 +156,11 @@ __global__ void __launch_bounds__(256) bonded_tuples(TupleArgs ta, const double 
     const double u = tuple_force(kind, xi, xj, xk, xl, p, box, f);
 #pragma unroll
     for (int k = 0; k < kTupleKinds; ++k) e[k] += k == kind ? u : 0.0;
-    add_force_words(F, place_of[a.x], f[0]);
-    add_force_words(F, place_of[a.y], f[1]);
-    if (kind >= kTupleAngle) add_force_words(F, place_of[a.z], f[2]);
-    if (kind >= kTupleDihedral) add_force_words(F, place_of[a.w], f[3]);
+    const auto at = [&](int atom) { return place_of ? place_of[atom] : atom; };
+    add_force_words(F, at(a.x), f[0]);
+    add_force_words(F, at(a.y), f[1]);
+    if (kind >= kTupleAngle) add_force_words(F, at(a.z), f[2]);
+    if (kind >= kTupleDihedral) add_force_words(F, at(a.w), f[3]);
   }
   if (ta.energy_partial) {
     for (int k = 0; k < kTupleKinds; ++k) {
@@ -174,6 +174,16 @@ __global__ void __launch_bounds__(256) bonded_tuples(TupleArgs ta, const double 
       __syncthreads();
     }
   }
+}
+
+// The tuples alone, into the place-ordered words (no PME beside them; with
+// PME they are the first blocks of pme_bin_tuples).
+__global__ void __launch_bounds__(256) bonded_tuples(TupleArgs ta, const double *__restrict__ x,
+                                                     const int *__restrict__ place_of,
+                                                     double bx, double by, double bz,
+                                                     long long *__restrict__ F) {
+  const double box[3] = {bx, by, bz};
+  tuple_block(blockIdx.x, gridDim.x, ta, x, place_of, box, F);
 }
 
 }  // namespace mdhip

@@ -1232,6 +1232,19 @@ struct Engine {
     launch_prune();
   }
 
+  // With PME in atom order beside the pairs the tuples run in its first
+  // launch, else before the pair loop.
+  bool tuples_in_bins() const { return use_pme && pme_atoms && (terms & 4); }
+  TupleArgs tuple_args(bool energy) const {
+    TupleArgs ta{};
+    ta.ntuples = ntuples;
+    ta.atoms = d_tuple_atoms;
+    ta.kind = d_tuple_kind;
+    ta.param = d_tuple_param;
+    ta.energy_partial = energy ? d_etup : nullptr;
+    return ta;
+  }
+
   // One launch: plane y = 0 of the grid takes the excluded and 1-4 pairs,
   // the planes above the segments of the group rows.
   template <int MOD, bool COUL, bool ENERGY, bool ORG>
@@ -1248,15 +1261,9 @@ struct Engine {
     sa.place_of = d_place_of;
     sa.energy_partial = ENERGY ? d_espec : nullptr;
     sa.p = spp;
-    if (const int tb = tuple_blocks()) {
-      TupleArgs ta{};
-      ta.ntuples = ntuples;
-      ta.atoms = d_tuple_atoms;
-      ta.kind = d_tuple_kind;
-      ta.param = d_tuple_param;
-      ta.energy_partial = ENERGY ? d_etup : nullptr;
-      bonded_tuples<<<tb, 256, 0, lstream>>>(ta, d_x, d_place_of, box[0], box[1], box[2], d_F);
-    }
+    if (const int tb = tuples_in_bins() ? 0 : tuple_blocks())
+      bonded_tuples<<<tb, 256, 0, lstream>>>(tuple_args(ENERGY), d_x, d_place_of, box[0], box[1],
+                                             box[2], d_F);
     const dim3 grid(std::max(blocks_for(max_groups, 4), blocks_for(nspecial)),
                     (terms & 1) ? nseg() + 1 : 1, nz);
     const bool pruned = prune_skin > 0;
@@ -1350,23 +1357,28 @@ struct Engine {
 
   // Lists the atoms of every brick their stencils touch.
   template <int N, int TL>
-  void bin_t() {
+  void bin_t(bool energy) {
+    if (const int tb = tuples_in_bins() ? tuple_blocks() : 0) {
+      pme_bin_tuples<N, TL><<<tb + blocks_for(n), 256, 0, pstream>>>(
+          d_pme_n, pme_positions(), pmp, bp, d_flags, tuple_args(energy), tb, d_x, d_Fr);
+      return;
+    }
     pme_bin<N, TL><<<dim3(blocks_for(pme_atoms ? n : max_places), 1, nz), 256, 0, pstream>>>(
         pme_atoms ? d_pme_n : d_counts, pme_positions(), pmp, bp, d_flags, fs);
   }
   template <int N>
-  void bin_n() {
+  void bin_n(bool energy) {
     switch (brick_tl) {
-      case 8: bin_t<N, 8>(); break;
-      case 4: bin_t<N, 4>(); break;
-      case 2: bin_t<N, 2>(); break;
-      default: bin_t<N, 1>(); break;
+      case 8: bin_t<N, 8>(energy); break;
+      case 4: bin_t<N, 4>(energy); break;
+      case 2: bin_t<N, 2>(energy); break;
+      default: bin_t<N, 1>(energy); break;
     }
   }
-  void pme_bin_launch() {
-    if (pme_order == 4) bin_n<4>();
-    else if (pme_order == 6) bin_n<6>();
-    else bin_n<8>();
+  void pme_bin_launch(bool energy = false) {
+    if (pme_order == 4) bin_n<4>(energy);
+    else if (pme_order == 6) bin_n<6>(energy);
+    else bin_n<8>(energy);
   }
 
   template <int N, int TL>
@@ -1596,7 +1608,7 @@ struct Engine {
 
   void pme(bool energy) {
     if (!use_pme) return;
-    pme_bin_launch();
+    pme_bin_launch(energy);
     pme_spread_launch();
     pme_yx(energy);
     pme_gather_rows_launch();

@@ -125,10 +125,9 @@ __device__ __forceinline__ void stencil_bricks(int f, int K, int nb, int &first,
 // run; nothing downstream depends on it).
 constexpr int kBinLdsBricks = 8192;
 template <int N, int TL>
-__global__ void __launch_bounds__(256) pme_bin(const int *__restrict__ counts,
-                                               const double4 *__restrict__ xpq,
-                                               PmeParams pp, BrickParams bp,
-                                               int *__restrict__ flags, size_t fs) {
+__device__ __forceinline__ void bin_block(int block, const int *__restrict__ counts,
+                                          const double4 *__restrict__ xpq, const PmeParams &pp,
+                                          BrickParams bp, int *__restrict__ flags, size_t fs) {
   constexpr int BX = BrickShape<TL>::BX, BY = BrickShape<TL>::BY;
   __shared__ int s_count[kBinLdsBricks];
   counts = frame_at(counts, fs);
@@ -140,7 +139,7 @@ __global__ void __launch_bounds__(256) pme_bin(const int *__restrict__ counts,
   const bool lds = nbricks <= kBinLdsBricks;
   if (lds)
     for (int k = threadIdx.x; k < nbricks; k += blockDim.x) s_count[k] = 0;
-  const int place = blockIdx.x * blockDim.x + threadIdx.x;
+  const int place = block * blockDim.x + threadIdx.x;
   // at most this many bricks per axis: whole ones, one more at each end, a
   // partial one at the wrap
   constexpr int MX = (N - 2) / BX + 3 < N ? (N - 2) / BX + 3 : N;
@@ -189,6 +188,31 @@ __global__ void __launch_bounds__(256) pme_bin(const int *__restrict__ counts,
       else
         atomicOr(&flags[kFlagBrickOverflow], 1);
     }
+}
+
+template <int N, int TL>
+__global__ void __launch_bounds__(256) pme_bin(const int *__restrict__ counts,
+                                               const double4 *__restrict__ xpq,
+                                               PmeParams pp, BrickParams bp,
+                                               int *__restrict__ flags, size_t fs) {
+  bin_block<N, TL>(blockIdx.x, counts, xpq, pp, bp, flags, fs);
+}
+
+// The bonded tuples as the launch's first `tuples` blocks, then the bins:
+// both read only what the integration wrote by atom (x and xpa), so the
+// tuples' forces go to the reciprocal part's words by atom (Fr) and neither
+// waits for a list build.  A launch of their own before the pair loop (one
+// wave of f64 work per SIMD, 8.6 us at 25,000 atoms) lengthened the list
+// branch by that.
+template <int N, int TL>
+__global__ void __launch_bounds__(256) pme_bin_tuples(
+    const int *__restrict__ counts, const double4 *__restrict__ xpq, PmeParams pp,
+    BrickParams bp, int *__restrict__ flags, TupleArgs ta, int tuples,
+    const double *__restrict__ x, long long *__restrict__ Fr) {
+  if ((int)blockIdx.x < tuples)
+    tuple_block(blockIdx.x, tuples, ta, x, nullptr, pp.box, Fr);
+  else
+    bin_block<N, TL>(blockIdx.x - tuples, counts, xpq, pp, bp, flags, 0);
 }
 
 // The spread, the gather and their adjoints come with SP = 1 and SP = 2
@@ -870,6 +894,8 @@ template __global__ void fft_rows_r2c<float, true>(const void *, cpx<float> *, i
 #define MDHIP_SPREAD(N, TL)                                                              \
   template __global__ void pme_bin<N, TL>(const int *, const double4 *, PmeParams,       \
       BrickParams, int *, size_t);                                                       \
+  template __global__ void pme_bin_tuples<N, TL>(const int *, const double4 *,           \
+      PmeParams, BrickParams, int *, TupleArgs, int, const double *, long long *);       \
   MDHIP_SPREAD_SP(N, TL, 1) MDHIP_SPREAD_SP(N, TL, 2)
 #define MDHIP_SPREAD_N(N) MDHIP_SPREAD(N, 8) MDHIP_SPREAD(N, 4) MDHIP_SPREAD(N, 2) MDHIP_SPREAD(N, 1)
 MDHIP_SPREAD_N(4)
