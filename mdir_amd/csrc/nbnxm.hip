@@ -308,10 +308,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) n
     const int *__restrict__ col_cl_start, const int *__restrict__ col_cl_count,
     const int *__restrict__ atom_at, const int *__restrict__ place_of,
     const int *__restrict__ excl_start, const int *__restrict__ excl_atoms,
+    const float4 *__restrict__ xq, const float4 *__restrict__ gorig,
     const int *__restrict__ counts_in, int *__restrict__ col_count,
     PairEntry *__restrict__ rows, int *__restrict__ row_count,
     uint64_t *__restrict__ ex_masks, int ex_cap, int *__restrict__ flags,
-    GridParams g, size_t fs) {
+    GridParams g, int exact, size_t fs) {
+  xq = frame_at(xq, fs);
+  gorig = frame_at(gorig, fs);
   bb_lo = frame_at(bb_lo, fs);
   bb_hi = frame_at(bb_hi, fs);
   cluster_col = frame_at(cluster_col, fs);
@@ -385,9 +388,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) n
 #pragma unroll
   for (int m = 0; m < kGroup; ++m) group_real |= mreal[m];
   const bool any_real = group_real != 0u;
+  // the group's atoms for the test of atom pairs: this lane's of each member
+  float xi[kGroup][3];
+  float4 oi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (exact) {
+#pragma unroll
+    for (int m = 0; m < kGroup; ++m) {
+      const float4 p = xq[(g0 + m) * kCluster + (lane & 7)];
+      xi[m][0] = p.x;
+      xi[m][1] = p.y;
+      xi[m][2] = p.z;
+    }
+    oi = gorig[gi];
+  }
   const int icol = cluster_col[g0];
   const int cx = icol % g.ncx, cy = icol / g.ncx;
   const float Lx = (float)g.box[0], Ly = (float)g.box[1], Lz = (float)g.box[2];
+  const float Lx_lo = (float)(g.box[0] - (double)Lx), Ly_lo = (float)(g.box[1] - (double)Ly),
+              Lz_lo = (float)(g.box[2] - (double)Lz);
   const float wxf = (float)g.wx, wyf = (float)g.wy;
   const float zreach = sqrtf(g.rlist2) * 1.0001f + 1.0e-5f;
   const int ncolx = 2 * g.rx + 1, ncols = any_real ? ncolx * (2 * g.ry + 1) : 0;
@@ -531,7 +549,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) n
     for (int round = 0; round * kWaves < niter; ++round) {
       const int t = (round * kWaves + wave) * 64 + lane;
       uint32_t imask = 0, jreal = 0, scode = 0;
-      int cj = 0, ex = -1;
+      int cj = 0, ex = -1, lex = 0;   // lex: the sign of the shift, z first
       if (t < total) {
         // the column slot holding candidate t: last slot with cbase <= t
         int lo = 0, hi = 63;
@@ -553,7 +571,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) n
         cj = s_cstart[lo] + s_k0[sz + 1][lo] + within;
         const int ccode = s_ccode[lo];
         const int sx = (ccode & 3) - 1, sy = ((ccode >> 2) & 3) - 1;
-        const int lex = sz != 0 ? sz : (sy != 0 ? sy : sx);
+        lex = sz != 0 ? sz : (sy != 0 ? sy : sx);
         jreal = real_mask[cj];
         scode = (uint32_t)(sx + 1) | ((uint32_t)(sy + 1) << 2) | ((uint32_t)(sz + 1) << 4);
         if (jreal) {
@@ -570,6 +588,46 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) n
               imask |= 1u << m;
           }
         }
+      }
+      // With `exact`, only the members with an atom pair within the reach stay:
+      // the wave takes the candidates its lanes found by their boxes four at
+      // a time (their loads together), lane l the pair (l & 7, l >> 3) of
+      // each tile.
+      for (uint64_t rem = exact ? __ballot(imask != 0u) : 0ull; rem;) {
+        constexpr int kBatch = 4;
+        int src[kBatch];
+        float4 xj[kBatch], oj[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+          src[k] = rem ? __builtin_ctzll(rem) : -1;
+          rem &= rem - 1;   // 0 stays 0
+          const int cjk = __builtin_amdgcn_readlane(cj, src[k] < 0 ? src[0] : src[k]);
+          xj[k] = xq[cjk * kCluster + (lane >> 3)];
+          oj[k] = gorig[cjk / kGroup];
+        }
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+          if (src[k] < 0) continue;
+          const uint32_t im = __builtin_amdgcn_readlane(imask, src[k]);
+          const uint32_t sc = __builtin_amdgcn_readlane(scode, src[k]);
+          const uint32_t jr = __builtin_amdgcn_readlane(jreal, src[k]);
+          const float xjx = xj[k].x + group_offset(sc, 0, oj[k].x, oi.x, Lx, Lx_lo);
+          const float xjy = xj[k].y + group_offset(sc, 1, oj[k].y, oi.y, Ly, Ly_lo);
+          const float xjz = xj[k].z + group_offset(sc, 2, oj[k].z, oi.z, Lz, Lz_lo);
+          const bool jreal_b = (jr >> (lane >> 3)) & 1u;
+          uint32_t members = 0;
+#pragma unroll
+          for (int m = 0; m < kGroup; ++m) {
+            if (!((im >> m) & 1u)) continue;  // uniform
+            const float dx = xi[m][0] - xjx, dy = xi[m][1] - xjy, dz = xi[m][2] - xjz;
+            const bool near = jreal_b && ((mreal[m] >> (lane & 7)) & 1u) &&
+                              dx * dx + dy * dy + dz * dz < g.rlist2;
+            if (__ballot(near)) members |= 1u << m;
+          }
+          if (lane == src[k]) imask = members;
+        }
+      }
+      if (t < total) {
         if (imask) {
           // a tile of a member with itself, or one that holds excluded pairs
           const int self = cj - g0;
