@@ -297,8 +297,8 @@ __device__ __forceinline__ float axis_gap(float lo_i, float hi_i, float lo_j,
 // candidates each per round (wave w takes the round's iteration w), and a
 // block prefix over the waves places their entries, so the row holds the
 // candidates in their order, as one wave walking them would write it.  Bit
-// m of an entry's imask is set when j is within the reach of member m and
-// the tile (member, j, shift) is ordered, so that each unordered cluster
+// m of an entry's imask is set when j is within the reach of member m (by
+// the clusters' boxes; with `exact`, by a pair of their atoms) and the tile (member, j, shift) is ordered, so that each unordered cluster
 // pair occurs once.  Tiles of a cluster with itself, and tiles holding
 // excluded pairs, get four explicit 64-bit masks (MDExecKernels.cpp:1748-1823
 // removes the same partners from a matrix row).
