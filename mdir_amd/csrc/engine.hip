@@ -227,26 +227,29 @@ struct Engine {
   // entries per pair-loop segment (16, 24 or 48): short segments give one
   // system more waves to hide latency with; a batch of frames fills the
   // GPU with long ones (a launch shape, see autotune)
-  int seg_len = 16, seg_len_cfg = 0;
+  int seg_len = 16;
   // Entries one wave of the pair loops takes ("piece"): the segment, halved
   // (down to kPieceMin) while the launch would hold fewer than kFillPieces
   // pieces.  A wave walks its entries in series, and a small box has fewer
   // waves than the GPU has SIMDs: 864 argon atoms took 11.9 us for 16
-  // entries (50 steps 1,060 us), 4 entries take the 50 steps to 810 us.
-  // Pieces are counted by capacity, about three times the entries the rows
-  // hold: the line lies near 1,000 waters, below which PME is shorter than
-  // the pair loop.  A line at 16,384 (4,000 waters) gave nothing more alone
-  // and cost replicas, which share the GPU, 2 to 4 %.  Frame batches keep
-  // whole segments: a frame's forces have the same bits whatever batch it
-  // is in, and the sums over a piece are f32.
+  // entries (50 steps 1,032 us), 4 entries take the 50 steps to 766 us.
+  // Pieces are counted by the rows' estimated capacity (row_entries), about
+  // three times the entries the rows hold: the line lies near 1,000 waters,
+  // below which PME is shorter than the pair loop.  A line at 16,384 (4,000
+  // waters) gave nothing more alone and cost replicas, which share the GPU, 2
+  // to 4 %.  The estimate is one of n, the box and the reach, never of a
+  // capacity that has grown: the sums over a piece are f32, so a piece that
+  // depended on what the engine held before would change a restored run's
+  // bits.  Frame batches keep whole segments for the same reason: a frame's
+  // forces have the same bits whatever batch it is in.
   static constexpr int kPieceMin = 4;
   static constexpr double kFillPieces = 4096;
   bool split_segments = true;
+  double row_entries = 0;   // entries of all rows by configure_list's estimate
+  int piece_cfg = 0;        // the piece the list's buffers are laid out for
   int piece() const {
     int len = seg_len;
-    while (split_segments && len / 2 >= kPieceMin &&
-           (double)max_groups * g.row_cap / len < kFillPieces)
-      len /= 2;
+    while (split_segments && len / 2 >= kPieceMin && row_entries / len < kFillPieces) len /= 2;
     return len;
   }
   int nseg() const { return (g.row_cap + piece() - 1) / piece(); }  // pieces per row
@@ -750,19 +753,20 @@ struct Engine {
     double est = (ng.wx + 2 * rb) * (ng.wy + 2 * rb) *
                  (std::min(kGroup * h, box[2]) + 2 * rb) / (ng.wx * ng.wy * h);
     est = std::min(est, (double)ng.max_clusters * 3.0);
-    int rc_ = (int)(1.25 * est + 64);
-    rc_ = std::max(rc_, row_cap_min);
-    ng.row_cap = (rc_ + kSegmentMax - 1) / kSegmentMax * kSegmentMax;
+    const auto whole = [](int c) { return (c + kSegmentMax - 1) / kSegmentMax * kSegmentMax; };
+    const int rc_ = (int)(1.25 * est + 64);
+    row_entries = (double)ngroups_max * whole(rc_);
+    ng.row_cap = whole(std::max(rc_, row_cap_min));
     ng.max_excl = 16;
     const int nex = std::max(ex_cap_min, ngroups_max * 16 + 1024);
     const bool same = d_rows && ng.ncol == g.ncol && ng.col_cap == g.col_cap &&
                       ng.row_cap == g.row_cap && ng.max_clusters == g.max_clusters &&
-                      nex == ex_cap && seg_len == seg_len_cfg;
+                      nex == ex_cap && piece() == piece_cfg;
     g = ng;
     list_reach = reach;
     if (same) return;
     max_groups = ngroups_max;
-    seg_len_cfg = seg_len;
+    piece_cfg = piece();
     ex_cap = nex;
     release_list();
     max_places = g.max_clusters * kCluster;
@@ -2134,7 +2138,7 @@ struct Engine {
     if (len != 16 && len != 24 && len != 48)
       throw HipError("pair-loop segments: 16, 24 or 48 entries");
     seg_len = len;
-    if (d_rows && seg_len_cfg != len) configure_list(list_reach, g.col_cap, g.row_cap, ex_cap);
+    if (d_rows && piece_cfg != piece()) configure_list(list_reach, g.col_cap, g.row_cap, ex_cap);
   }
   // One launch shape, set directly (what the trial keeps can be set again
   // without timing): segment entries 16, 24 or 48; PME bricks of 8, 4, 2 or
