@@ -1222,11 +1222,11 @@ struct Engine {
   static constexpr int kExactAtoms = 64000;
   bool exact_search() const { return n >= kExactAtoms && !d_arena; }
   void launch_search() {
-    nb_search<<<dim3(max_groups, 1, nz), 256, 0, lstream>>>(
+    const auto kernel = exact_search() ? nb_search<true> : nb_search<false>;
+    kernel<<<dim3(max_groups, 1, nz), 256, 0, lstream>>>(
         d_bb_lo, d_bb_hi, d_cluster_col, d_real_mask, d_col_cl_start, d_col_cl_count,
         d_atom_at, d_place_of, d_excl_start, d_excl_atoms, d_xq, d_gorig, d_counts, d_col_count,
-        d_rows,
-        d_row_count, d_ex, ex_cap, d_flags, g, exact_search() ? 1 : 0, fs);
+        d_rows, d_row_count, d_ex, ex_cap, d_flags, g, fs);
   }
   void launch_prune() {
     if (prune_skin <= 0) return;

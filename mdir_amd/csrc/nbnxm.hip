@@ -298,10 +298,14 @@ __device__ __forceinline__ float axis_gap(float lo_i, float hi_i, float lo_j,
 // block prefix over the waves places their entries, so the row holds the
 // candidates in their order, as one wave walking them would write it.  Bit
 // m of an entry's imask is set when j is within the reach of member m (by
-// the clusters' boxes; with `exact`, by a pair of their atoms) and the tile (member, j, shift) is ordered, so that each unordered cluster
-// pair occurs once.  Tiles of a cluster with itself, and tiles holding
-// excluded pairs, get four explicit 64-bit masks (MDExecKernels.cpp:1748-1823
-// removes the same partners from a matrix row).
+// the clusters' boxes; EXACT: by a pair of their atoms) and the tile (member,
+// j, shift) is ordered, so that each unordered cluster pair occurs once.
+// Tiles of a cluster with itself, and tiles holding excluded pairs, get four
+// explicit 64-bit masks (MDExecKernels.cpp:1748-1823 removes the same partners
+// from a matrix row).  EXACT is a template argument because its test takes 80
+// registers where the plain form takes 61: two waves per SIMD that small boxes
+// and batches of frames, which never run the test, would lose.
+template <bool EXACT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) nb_search(
     const float4 *__restrict__ bb_lo, const float4 *__restrict__ bb_hi,
     const int *__restrict__ cluster_col, const uint32_t *__restrict__ real_mask,
@@ -312,9 +316,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) n
     const int *__restrict__ counts_in, int *__restrict__ col_count,
     PairEntry *__restrict__ rows, int *__restrict__ row_count,
     uint64_t *__restrict__ ex_masks, int ex_cap, int *__restrict__ flags,
-    GridParams g, int exact, size_t fs) {
-  xq = frame_at(xq, fs);
-  gorig = frame_at(gorig, fs);
+    GridParams g, size_t fs) {
+  if constexpr (EXACT) {
+    xq = frame_at(xq, fs);
+    gorig = frame_at(gorig, fs);
+  }
   bb_lo = frame_at(bb_lo, fs);
   bb_hi = frame_at(bb_hi, fs);
   cluster_col = frame_at(cluster_col, fs);
@@ -350,8 +356,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) n
   // the z bounds of the chunk's columns' clusters, staged so that the
   // binary searches read LDS instead of chains of dependent global loads
   // (chunks of more clusters read them from global memory).  1,024 keeps
-  // the block at 19 KB of LDS and, with 63 VGPRs, eight blocks fit a CU:
-  // a batch of frames launches thousands of these blocks.
+  // the block at 19 KB of LDS and, with the plain form's 61 VGPRs, eight
+  // blocks fit a CU: a batch of frames launches thousands of these blocks.
   constexpr int kZStage = 1024;
   __shared__ float s_zlo[kZStage], s_zhi[kZStage];
   __shared__ int s_zoff[64], s_zn[64], s_kmin[64];
@@ -391,7 +397,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) n
   // the group's atoms for the test of atom pairs: this lane's of each member
   float xi[kGroup][3];
   float4 oi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (exact) {
+  if constexpr (EXACT) {
 #pragma unroll
     for (int m = 0; m < kGroup; ++m) {
       const float4 p = xq[(g0 + m) * kCluster + (lane & 7)];
@@ -589,42 +595,43 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) n
           }
         }
       }
-      // With `exact`, only the members with an atom pair within the reach stay:
-      // the wave takes the candidates its lanes found by their boxes four at
-      // a time (their loads together), lane l the pair (l & 7, l >> 3) of
-      // each tile.
-      for (uint64_t rem = exact ? __ballot(imask != 0u) : 0ull; rem;) {
-        constexpr int kBatch = 4;
-        int src[kBatch];
-        float4 xj[kBatch], oj[kBatch];
+      if constexpr (EXACT) {
+        // only the members with an atom pair within the reach stay: the wave
+        // takes the candidates its lanes found by their boxes four at a time
+        // (their loads together), lane l the pair (l & 7, l >> 3) of each tile
+        for (uint64_t rem = __ballot(imask != 0u); rem;) {
+          constexpr int kBatch = 4;
+          int src[kBatch];
+          float4 xj[kBatch], oj[kBatch];
 #pragma unroll
-        for (int k = 0; k < kBatch; ++k) {
-          src[k] = rem ? __builtin_ctzll(rem) : -1;
-          rem &= rem - 1;   // 0 stays 0
-          const int cjk = __builtin_amdgcn_readlane(cj, src[k] < 0 ? src[0] : src[k]);
-          xj[k] = xq[cjk * kCluster + (lane >> 3)];
-          oj[k] = gorig[cjk / kGroup];
-        }
-#pragma unroll
-        for (int k = 0; k < kBatch; ++k) {
-          if (src[k] < 0) continue;
-          const uint32_t im = __builtin_amdgcn_readlane(imask, src[k]);
-          const uint32_t sc = __builtin_amdgcn_readlane(scode, src[k]);
-          const uint32_t jr = __builtin_amdgcn_readlane(jreal, src[k]);
-          const float xjx = xj[k].x + group_offset(sc, 0, oj[k].x, oi.x, Lx, Lx_lo);
-          const float xjy = xj[k].y + group_offset(sc, 1, oj[k].y, oi.y, Ly, Ly_lo);
-          const float xjz = xj[k].z + group_offset(sc, 2, oj[k].z, oi.z, Lz, Lz_lo);
-          const bool jreal_b = (jr >> (lane >> 3)) & 1u;
-          uint32_t members = 0;
-#pragma unroll
-          for (int m = 0; m < kGroup; ++m) {
-            if (!((im >> m) & 1u)) continue;  // uniform
-            const float dx = xi[m][0] - xjx, dy = xi[m][1] - xjy, dz = xi[m][2] - xjz;
-            const bool near = jreal_b && ((mreal[m] >> (lane & 7)) & 1u) &&
-                              dx * dx + dy * dy + dz * dz < g.rlist2;
-            if (__ballot(near)) members |= 1u << m;
+          for (int k = 0; k < kBatch; ++k) {
+            src[k] = rem ? __builtin_ctzll(rem) : -1;
+            rem &= rem - 1;   // 0 stays 0
+            const int cjk = __builtin_amdgcn_readlane(cj, src[k] < 0 ? src[0] : src[k]);
+            xj[k] = xq[cjk * kCluster + (lane >> 3)];
+            oj[k] = gorig[cjk / kGroup];
           }
-          if (lane == src[k]) imask = members;
+#pragma unroll
+          for (int k = 0; k < kBatch; ++k) {
+            if (src[k] < 0) continue;
+            const uint32_t im = __builtin_amdgcn_readlane(imask, src[k]);
+            const uint32_t sc = __builtin_amdgcn_readlane(scode, src[k]);
+            const uint32_t jr = __builtin_amdgcn_readlane(jreal, src[k]);
+            const float xjx = xj[k].x + group_offset(sc, 0, oj[k].x, oi.x, Lx, Lx_lo);
+            const float xjy = xj[k].y + group_offset(sc, 1, oj[k].y, oi.y, Ly, Ly_lo);
+            const float xjz = xj[k].z + group_offset(sc, 2, oj[k].z, oi.z, Lz, Lz_lo);
+            const bool jreal_b = (jr >> (lane >> 3)) & 1u;
+            uint32_t members = 0;
+#pragma unroll
+            for (int m = 0; m < kGroup; ++m) {
+              if (!((im >> m) & 1u)) continue;  // uniform
+              const float dx = xi[m][0] - xjx, dy = xi[m][1] - xjy, dz = xi[m][2] - xjz;
+              const bool near = jreal_b && ((mreal[m] >> (lane & 7)) & 1u) &&
+                                dx * dx + dy * dy + dz * dz < g.rlist2;
+              if (__ballot(near)) members |= 1u << m;
+            }
+            if (lane == src[k]) imask = members;
+          }
         }
       }
       if (t < total) {
