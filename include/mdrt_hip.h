@@ -329,9 +329,11 @@ int mdrtHipComputeForceTerms(void *system, int32_t terms, double *forces, double
 int mdrtHipSetPmeTransform(void *system, int32_t mode);
 
 /* One launch shape, set directly (as the trial below would keep it):
-   pair-loop segments of 16, 24 or 48 row entries, PME bricks of 8, 4, 2 or
-   1 complex z lines (those that fit LDS at this grid), plane transform 0 or
-   1 (as mdrtHipSetPmeTransform). The list is rebuilt at the next
+   pair-loop segments of 16, 24 or 48 row entries (the most a wave takes: in
+   boxes too small to fill the GPU with such segments a wave takes a half, a
+   quarter or an eighth of one, so that lengths may come down to the same
+   launch), PME bricks of 8, 4, 2 or 1 complex z lines (those that fit LDS at
+   this grid), plane transform 0 or 1 (as mdrtHipSetPmeTransform). The list is rebuilt at the next
    evaluation. The counterpart of a launch shape chosen in the reference's
    TOWERS set-up (tools/mdir/TowersShape.h). */
 int mdrtHipSetLaunchShape(void *system, int32_t segment, int32_t bricks, int32_t transform);
@@ -346,15 +348,16 @@ int mdrtHipGetLaunchShape(void *system, int32_t *shape);
    Run.cpp:913-926). Bit 0 of `what`: PME bricks of 8, 4, 2 or 1 complex z
    lines (those that fit LDS). Bit 1: the plane transform (0 or 1 of
    mdrtHipSetPmeTransform, where the grid allows 1). Bit 2: pair-loop
-   segments of 16, 24 or 48 row entries per wave. Each candidate runs one
-   untimed captured graph of `steps` steps of dt (ps), then `graphs` timed
-   ones, from the same positions and velocities, which are restored at the
-   end; two passes over the candidates, the faster time of each counting,
-   and the current shape stays unless another is 2 % faster.
+   segments of at most 16, 24 or 48 row entries per wave. Each candidate
+   runs one untimed captured graph of `steps` steps of dt (ps), then
+   `graphs` timed ones, from the same positions and velocities, which are
+   restored at the end; two passes over the candidates, the faster time of
+   each counting, and the current shape stays unless another is 2 % faster.
    ms_per_step[24]: [8 * s + 4 * transform + k] for segments of 16, 24, 48
-   (s = 0, 1, 2) and bricks of TL = 8 >> k, NaN for shapes not run. The
-   shapes give the same forces up to the f32 rounding of the gather's
-   per-brick partial sums (up to about 1e-7 relative). */
+   (s = 0, 1, 2) and bricks of TL = 8 >> k, NaN for shapes not run; segment
+   lengths that are the same launch in this box are run once and share the
+   time. The shapes give the same forces up to the f32 rounding of the
+   gather's per-brick partial sums (up to about 1e-7 relative). */
 int mdrtHipAutotune(void *system, int32_t what, int32_t steps, int32_t graphs, double dt,
                     double *ms_per_step);
 

@@ -247,11 +247,11 @@ struct Engine {
   bool split_segments = true;
   double row_entries = 0;   // entries of all rows by configure_list's estimate
   int piece_cfg = 0;        // the piece the list's buffers are laid out for
-  int piece() const {
-    int len = seg_len;
+  int piece_of(int len) const {
     while (split_segments && len / 2 >= kPieceMin && row_entries / len < kFillPieces) len /= 2;
     return len;
   }
+  int piece() const { return piece_of(seg_len); }
   int nseg() const { return (g.row_cap + piece() - 1) / piece(); }  // pieces per row
   int *d_excl_start = nullptr, *d_excl_atoms = nullptr;
   int *d_flags = nullptr;
@@ -2112,16 +2112,26 @@ struct Engine {
     return c;
   }
   // Runs measure(shape) for every candidate in two passes, fills ms_out
-  // with the faster time of each, and returns the shape to keep.
+  // with the faster time of each, and returns the shape to keep.  Segment
+  // lengths that come down to the same piece in this box are one shape: the
+  // first is run, and its time stands for all of them.
   template <class Measure>
-  static Shape trial(const std::vector<Shape> &cands, Shape cur, Measure measure,
-                     double *ms_out) {
+  Shape trial(const std::vector<Shape> &cands, Shape cur, Measure measure,
+              double *ms_out) const {
+    const auto first_alike = [&](const Shape &c) {
+      for (const Shape &o : cands)
+        if (o.tr == c.tr && o.k == c.k && piece_of(kSegLens[o.s]) == piece_of(kSegLens[c.s]))
+          return o;
+      return c;
+    };
     for (int pass = 0; pass < 2; ++pass)
       for (const Shape &c : cands) {
+        if (first_alike(c).s != c.s) continue;
         const double ms = measure(c);
         double &slot = ms_out[c.slot()];
         slot = std::isnan(slot) ? ms : std::min(slot, ms);
       }
+    for (const Shape &c : cands) ms_out[c.slot()] = ms_out[first_alike(c).slot()];
     Shape best = cur;
     bool have = false, cur_in = false;
     for (const Shape &c : cands) {

@@ -710,7 +710,7 @@ struct FrameBatch {
     auto call = [&]() {
       force_matching(frames, positions, f_ref, loss.data(), dq.data(), ds.data(), de.data(), 1);
     };
-    const Engine::Shape keep = Engine::trial(
+    const Engine::Shape keep = e.trial(
         Engine::trial_shapes(what, e.use_pme ? e.pme_grid[2] : 0, mfma_ok, tl0, tr0, e.seg_len),
         cur,
         [&](const Engine::Shape &c) {

@@ -126,7 +126,8 @@ class Simulation:
 
     @property
     def launch_shape(self) -> tuple:
-        """(segment entries, PME brick z lines, plane transform)."""
+        """(segment entries, PME brick z lines, plane transform).  The entries
+        are the most one wave takes; small boxes share a segment among waves."""
         out = np.zeros(3, np.int32)
         rt.check(rt.lib().mdrtHipGetLaunchShape(self._h, rt.ptr(out, C.c_int32)))
         return tuple(int(v) for v in out)
