@@ -827,8 +827,10 @@ __global__ void __launch_bounds__(512) nb_prune(
 
 // For every tile lane with its mask bit set, the reference matrix test of
 // NeighborsMatrix.mlir:176-183 and :394-412 on positions wrapped in f64 and
-// rounded to f32 (each operation rounded on its own); pairs that pass are
-// written as (min atom, max atom).  The host removes duplicates.
+// rounded to f32; pairs that pass are written as (min atom, max atom).  The
+// host removes duplicates.  Each operation is rounded on its own: plain
+// operators under contract(off), since HIP's __fmul_rn and __fadd_rn are
+// operators of a header where products still fuse into sums.
 __global__ void __launch_bounds__(256) nb_export_pairs(
     const double *__restrict__ x, const int *__restrict__ atom_at,
     const uint32_t *__restrict__ real_mask, const PairEntry *__restrict__ rows,
@@ -841,8 +843,7 @@ __global__ void __launch_bounds__(256) nb_export_pairs(
   const int gi = blockIdx.x * 4 + wave;
   if (gi >= counts_in[1] / kGroup) return;
   const int a = lane & 7, b = lane >> 3;
-  const float ilx = __fdiv_rn(1.0f, Lx), ily = __fdiv_rn(1.0f, Ly),
-              ilz = __fdiv_rn(1.0f, Lz);
+  const float ilx = 1.0f / Lx, ily = 1.0f / Ly, ilz = 1.0f / Lz;
   const double L[3] = {bx, by, bz};
   const float Lf[3] = {Lx, Ly, Lz}, il[3] = {ilx, ily, ilz};
   const int n = row_count[gi];
@@ -871,14 +872,14 @@ __global__ void __launch_bounds__(256) nb_export_pairs(
       }
       float d2[3];
       for (int k = 0; k < 3; ++k) {
-        const float d = __fsub_rn(wi[k], wj[k]);
-        const float images = __fmul_rn(d, il[k]);
+        const float d = wi[k] - wj[k];
+        const float images = d * il[k];
         const float nearest = rintf(images);
-        const float sh = __fmul_rn(nearest, Lf[k]);
-        const float dd = __fsub_rn(d, sh);
-        d2[k] = __fmul_rn(dd, dd);
+        const float sh = nearest * Lf[k];
+        const float dd = d - sh;
+        d2[k] = dd * dd;
       }
-      const float r2 = __fadd_rn(__fadd_rn(d2[0], d2[1]), d2[2]);
+      const float r2 = (d2[0] + d2[1]) + d2[2];
       if (r2 < limit2) {
         const unsigned long long slot = atomicAdd(out_count, 1ull);
         if (slot < capacity) out[slot] = make_int2(ia < jb ? ia : jb, ia < jb ? jb : ia);
