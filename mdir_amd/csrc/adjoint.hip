@@ -684,6 +684,8 @@ __global__ void __launch_bounds__(256) nb_adjoint(
 
 // ---- PME: the dipole grid and the gathers ---------------------------------
 
+#pragma clang fp contract(on)   // as the stencils of pme.hip
+
 // B-spline second derivatives in u at the stencil points (the second
 // difference of the order n-2 weights: M_n'' = M_{n-2}(u) - 2 M_{n-2}(u-1)
 // + M_{n-2}(u-2), PMECode.h's recursion run to order n-2).
@@ -771,6 +773,8 @@ __device__ __forceinline__ void spread_dipole_atom(double4 pq, float4 c, int hal
   }
 }
 
+#pragma clang fp contract(fast)
+
 // The dipole grid of the cotangent, spread by the bricks of pme_bin's lists
 // and transformed along z like pme_spread_rows.
 template <int N, int TL, int SP>
@@ -805,6 +809,8 @@ __global__ void __launch_bounds__(SP * kBrickThreads) pme_spread_dipole(
   __syncthreads();
   brick_forward_z<TL>(acc, a, b, tw, az, pp, bp, bx0, by0, out);
 }
+
+#pragma clang fp contract(on)
 
 // Gathers of the potential phi (the forward's convolved grid) and psi (the
 // convolved dipole grid) at one atom, with q, the scaled cotangent c and
@@ -914,6 +920,8 @@ __device__ __forceinline__ void gather_adj_atom(double4 pq, float4 c, float gs, 
 #pragma unroll
   for (int k = 0; k < words; ++k) atomicAdd(u + k, (unsigned long long)wd[k]);
 }
+
+#pragma clang fp contract(fast)
 
 template <int N, int TL, int SP, int KIND>
 __global__ void __launch_bounds__(SP * kBrickThreads) pme_gather_adj(

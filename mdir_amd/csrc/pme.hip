@@ -31,6 +31,13 @@ struct PmeParams {
   double inv_box[3];
 };
 
+// The arithmetic of an atom's stencil (weights, spread, gather, and their
+// adjoints in adjoint.hip) fuses products into sums where an expression says
+// so, not where the code around an instance happens to allow it: instances
+// with one and with two threads to an atom then give the same bits, which a
+// frame in batches of different sizes needs.
+#pragma clang fp contract(on)
+
 // B-spline weights M[t] of the points first + t, t = 0..n-1, and their
 // derivatives in u, for fraction w (recursion of PMECode.h:147-186; closed
 // forms of 05-electrostatics.md:290 at order 4).
@@ -80,6 +87,8 @@ __device__ __forceinline__ void pme_place(double x, double L, double invL, int K
   if (f < 0) f += K;
   first = f;
 }
+
+#pragma clang fp contract(fast)
 
 // ---- spread fused with the forward z transform ---------------------------
 //
@@ -238,6 +247,8 @@ __device__ __forceinline__ unsigned long long grid_word(float p) {
   return (unsigned long long)__double2ll_rn((double)p * kGridScale);
 }
 
+#pragma clang fp contract(on)
+
 // The x planes `half`, half + SP, .. of one atom's stencil (first
 // points f, weights M, charge q), the part that lies in the brick at (bx0,
 // by0), added to the brick's accumulators.  SMALL: every product is below
@@ -294,6 +305,8 @@ __device__ __forceinline__ void spread_atom(double4 pq, int half, const PmeParam
   else
     spread_part<N, BX, BY, SP, false>(f, M, qf, half, pp, bx0, by0, acc);
 }
+
+#pragma clang fp contract(fast)
 
 // The brick's R accumulated real rows (64-bit words in acc) to their half
 // spectra along z in `out`: rows 2t and 2t+1 as the real and imaginary
@@ -386,6 +399,8 @@ __global__ void __launch_bounds__(SP * kBrickThreads) pme_spread_rows(
 // depend on the order of the adds).  The real potential grid never goes to
 // HBM.  The block clears its brick's list count for the next step.
 
+#pragma clang fp contract(on)
+
 // One atom's force from the potential rows of the brick at (bx0, by0):
 // -q (K/L) sum phi M' M M over the stencil points in the brick, summed over
 // the SP neighbouring threads that share the atom and added as
@@ -461,6 +476,8 @@ __device__ __forceinline__ void gather_atom(double4 pq, int half, int place, con
   atomicAdd(u + 1, (unsigned long long)w1);
   atomicAdd(u + 2, (unsigned long long)w2);
 }
+
+#pragma clang fp contract(fast)
 
 // The brick's half-spectrum rows of `in` back to real rows in LDS (one
 // complex line t per pair of rows 2t, 2t+1): returns the buffer (a or b)
