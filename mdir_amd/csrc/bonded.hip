@@ -8,12 +8,14 @@
 //   dihedral             k (1 + cos(n phi - phase))  phi of i-j-k-l, IUPAC
 //   harmonic improper    (k/2) wrap(phi - phi0)^2    wrap to [-pi, pi)
 //
-// Differences use the minimum image.  The forces go to the 64-bit words of
-// the atoms' places, as the excluded and 1-4 pairs' do; the kernel runs on
-// the list's stream after the build of the step has placed the atoms, as a
-// launch of its own (its f64 registers would lower the pair kernel's
-// occupancy were it a part of that launch).  The tuples are sorted by kind,
-// so a wave mostly runs one kind.
+// Differences use the minimum image.  With PME the tuples are the first
+// blocks of the bins' launch (pme_bin_tuples), beside the list build, and add
+// to the 64-bit words by atom.  Without PME, or where its terms are not asked
+// for, they are a launch of their own on the list's stream after the build of
+// the step has placed the atoms, and add to the words of the atoms' places, as
+// the excluded and 1-4 pairs do (inside the pair kernel's launch their f64
+// registers would lower its occupancy).  The tuples are sorted by kind, so a
+// wave mostly runs one kind.
 namespace mdhip {
 
 enum TupleKind { kTupleBond = 0, kTupleUreyBradley = 1, kTupleAngle = 2, kTupleDihedral = 3,

@@ -1216,9 +1216,12 @@ struct Engine {
   // Large boxes drop the tiles whose boxes are within the reach but no atom
   // pair is.  The pair loop, which they spend every step on, takes 137.7
   // instead of 156.1 us at 107,000 atoms and 1,033 instead of 1,188 us at
-  // 999,000; a search takes 10 to 20 % longer.  Below, a rebuild step waits
-  // for its search and the PME branch is as long as the pair loop: 50 steps
-  // of 24,000 atoms 4,150 to 4,240 us, of 1,500 atoms 2,500 to 2,800 us.
+  // 999,000; the mean search launch, empty ones among them, takes 20 to 40 %
+  // longer.  Below, a rebuild step waits for its search and the PME branch is
+  // as long as the pair loop.  50 steps
+  // without and with the test: 4,075 and 4,235 us at 24,000 atoms, 5,440 and
+  // 5,535 at 36,000, 7,180 and 7,170 at 53,000, 9,565 and 9,280 at 80,000,
+  // 12,365 and 12,015 at 107,000.
   static constexpr int kExactAtoms = 64000;
   bool exact_search() const { return n >= kExactAtoms && !d_arena; }
   void launch_search() {
@@ -1363,7 +1366,10 @@ struct Engine {
   // 4,487, 4,522, 4,317 us.  At 2,916 blocks (999,000 atoms) the spread
   // alone is faster still (176, 142, 115 us), but the larger blocks wait for
   // room beside the pair loop: a pass of 114.0, 112.7, 124.0 ms; 64 frames
-  // (4,096 blocks) 925, 922, 1,016 us.
+  // (4,096 blocks) 925, 922, 1,016 us.  Around the line, 20 steps with SP = 1
+  // and 2: 7,895 and 7,560 us at 1,024 blocks (190,000 atoms), 9,055 and 9,025
+  // at 1,280, 13,860 and 14,615 at 1,600.  Replicas of 36 to 196 blocks each,
+  // 64 or 128 on the GPU, give the same either way (4,063 and 4,095 ns/day).
   static constexpr int kSplitBlocks = 1024;
   int brick_split() const { return nbricks * nz <= kSplitBlocks ? 2 : 1; }
   const double4 *pme_positions() const { return pme_atoms ? d_xpa : d_xpq; }

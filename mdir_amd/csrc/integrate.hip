@@ -170,8 +170,8 @@ __device__ void settle_velocities(const double *xa, const double *xb, const doub
 }
 
 // The state of one unit of S atoms (a SETTLE water, S = 3, a constraint
-// cluster, S = 2..5, with its centre at index 0) in registers: S is a compile-time constant so that the arrays stay in
-// registers.
+// cluster, S = 2..5, with its centre at index 0): S is a compile-time constant
+// so that the arrays stay in registers.
 template <int S>
 struct UnitState {
   double im[S], x[S][3], v[S][3];
@@ -422,7 +422,9 @@ constexpr int kClusterUnits = kIntThreads / kClusterSlots;
 // a launch alone: 11.9 us at 14,000 atoms (a thread per unit, with a step
 // counter that every block advanced behind a fence: 18.2), 90 us at
 // 999,000 (520; 300 bytes an atom, 3.3 TB/s); 9.5 us without noise at
-// 24,000 (11.8).
+// 24,000 (11.8).  Beside waters a free atom takes the three slots of a unit:
+// 16.4 us for 79,000 of them and one water, 12.6 us in a system of free
+// atoms alone (a thread per unit: 64 and 57).
 template <int PART, bool CL>
 __global__ void __launch_bounds__(kIntThreads) integrate_units(
     IntUnits un, double *__restrict__ x, double *__restrict__ v,
@@ -621,7 +623,7 @@ __global__ void pme_pack_atoms(int n, const double *__restrict__ x, const double
 
 // The pair loop's f32 positions (and the f64 ones of PME in place order) of
 // every atom at its place in the current list, from x: the values a drift
-// stores (store_drifted, the same expressions without contraction), for
+// stores (integrate_units, the same expressions without contraction), for
 // positions set outside the steps while the list stays.
 __global__ void refresh_places(int n, const double *__restrict__ x,
                                const double *__restrict__ shift, const double *__restrict__ q,
